@@ -154,6 +154,7 @@ int gemv(int bits, const void* x, int m, int nseg, const void* const* wt, const 
     if (n[i] < 1 || !wt[i] || !st[i] || !y[i] || (ldy && ldy[i] < n[i])) return AK_INVALID;
   const bool exact = bf16w || (!force_default && exact_mode());
   if (act && exact) return AK_INVALID;  // the fused activation is in the default path's kernels only
+  std::lock_guard<std::mutex> lock(scratch_mutex(s));
   if (mm_route(m, k, group, exact)) {  // above the crossover: the fp16-MFMA kernel, all tokens at once
     const int e = mm_gemv(bits, x, m, make_segs(nseg, wt, st, y, n, ldy, 16), k, group, s, act);
     if (e != AK_INVALID) return e;

@@ -12,6 +12,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
+
 namespace agq {
 
 constexpr int kMaxSegs = 4;
@@ -39,6 +41,10 @@ struct ScratchOverride {
   bool on = false;
 };
 ScratchOverride& scratch_override();
+
+// Held while a call on stream s enqueues kernels that work in the stream's scratch: calls of two host threads on one
+// stream are then ordered as wholes, also those whose kernels hand data to each other through the scratch.
+std::mutex& scratch_mutex(hipStream_t s);
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));

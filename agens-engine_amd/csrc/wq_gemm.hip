@@ -7,30 +7,33 @@
 // and written to LDS, and v_mfma_f32_16x16x32_bf16 consumes them there: no dequantized copy, no second pass over the
 // weights (narrow linears split k across workgroups, with fp32 partials in the stream's split-K scratch).
 //
-// Two tilings, one kernel template (wq_gemm_kernel<BITS, G, R, T, RING, XR, XM, DMA>); k is walked in 64-input slabs.
-//   - 128 x 128 (R = T = 128; 256 threads, 4 waves, two workgroups per CU), where few tiles exist (narrow linears):
-//     thread (row tid / 2, half tid % 2) loads its lane chunk of the slab from the row's KT record (W4 16 B, W3
-//     8 + 4 B, W2 8 B) and the group's scale, RING - 1 slabs ahead in a ring of registers; the inputs are 1024 16-byte
-//     chunks per slab, 8 consecutive threads reading one token's 128 bytes, XR - 1 slabs ahead; both are written to
-//     two LDS stages (16 KB weights, dequantized, + 16 KB inputs).  Grid: row tile major with the token tiles of a row
-//     tile 8 workgroups apart (same XCD: workgroup i runs on XCD i % 8), sharing the row tile's weights in that L2.
-//   - 256 x 256 (R = T = 256; 512 threads, 8 waves, one workgroup per CU), where the tiles fill the GPU (wide linears,
-//     or from 2048 tokens): each weight is dequantized once per 256 tokens.  The tokens go straight from the buffer
-//     into LDS (buffer loads into LDS, two stages of 32 KB, one slab ahead; no registers), the weights through a
-//     register ring (W4 / W2 3 slabs ahead, W3 1) into two 32 KB stages; the next slab's dequantization is
-//     interleaved with this slab's MFMAs (after each 16 MFMAs one of its four words; one MFMA, three VALU instructions
-//     alternating), since the two waves of a SIMD leave the slab's barrier together.  Grid: the tiles in token-major order cut into 8
-//     contiguous runs, XCD x taking run x, so that each XCD works on one or two token tiles (256 tokens x k inputs)
-//     that stay in its L2 while the weights stream.
-// Common: raw buffer loads with a per-lane offset fixed for the kernel and a scalar per-slab offset keep address
-// arithmetic off the vector unit; no load sits under a branch (the compiler's wait counts stay exact).  LDS rows /
-// tokens of 64 bf16 (128 B): the 16-byte chunk q of row r sits at slot q ^ ((r >> 1) & 7), so the 16 rows of one MFMA
-// operand read hit 16 distinct 16-byte bank slots.  Wave tiles of 64 rows x 64 (128 x 128) or 128 (256 x 256)
-// tokens, 16 x 16 MFMA tiles, two 32-input slices per slab; lane l reads 8 inputs 8 (l / 16) .. of its slice for row /
-// token l % 16 (the same input-to-slot map for weights and tokens, which is all an MFMA needs).
-// The accumulation order is this kernel's own (fp32 MFMA sums over 32 inputs, slabs in order): results agree with the
+// Tiling: 256 output rows x T tokens (T = 64, 128, 192, 256, by pick_tiling) per workgroup of 8 waves, wave tiles of 64
+// rows x T / 2 tokens as 32 x 32 MFMA tiles, k in slabs of 64 inputs.  Thread (row tid / 2, half tid % 2) loads its lane
+// chunk of the slab from the row's KT record (W4 16 B, W3 8 + 4 B, W2 8 B) and the group's scale three slabs ahead into
+// one of two register sets; the tokens go straight from the buffer into LDS (buffer loads into LDS, two stages, two
+// slabs ahead); the weights are dequantized once per T tokens into two 32 KB LDS stages.
+// What bounds it: per slab a SIMD's two waves need 2048 cycles of MFMA at T = 256, the workgroup's operand reads and
+// writes the LDS for as long, and the dequantization about 1400 cycles of each SIMD's VALU; each is hidden behind the
+// others only if no wave waits for its own.  So the slab is pipelined in slices of 16 inputs: the operands of a slice (24
+// registers with 32 x 32 tiles) are read from LDS while the MFMAs of the slice before run, with a quarter or half of the
+// next slab's dequantization mixed in (sched_group_barrier); the slab's barrier stands before its last slice's MFMAs,
+// whose operands every wave already holds, so that the next slab's first operands are read behind them and the stage
+// just left is free for the DMA of two slabs ahead.  The waits on global loads are counted: the token loads of the next
+// slab, not the weights of the one after.
+// Measured (us, before = 16 x 16 MFMA tiles with each slice's operands read right before its MFMAs): gate_up 55296 x
+// 5120 W3 at 512 tokens 334 -> 283, 300 tokens 326 -> 229 (T = 192), 2048 tokens 1172 -> 1049; o 5120 x 5120 W4 at 256
+// tokens 41 -> 31; down 5120 x 27648 W2 at 333 tokens 162 -> 112; 1.0-1.1 PFLOP/s where a round of tiles is full.
+// Grid: the items (split, token tile, row tile) in that order cut into 8 contiguous runs, XCD x (workgroup i runs on XCD
+// i % 8) taking run x, so that each XCD works on one or two token tiles (T tokens x k inputs) that stay in its L2 while
+// the weights stream, and every XCD has as many workgroups as the others.
+// Raw buffer loads with a per-lane offset fixed for the kernel and a scalar per-slab offset keep address arithmetic off
+// the vector unit; no load sits under a branch (the compiler's wait counts stay exact).  LDS rows / tokens of 64 bf16
+// (128 B): the 16-byte chunk q of row r sits at slot q ^ ((r >> 1) & 7), so 16 rows of an MFMA operand read hit 16
+// distinct 16-byte bank slots.  Lane l reads 8 inputs 8 (l / 32) .. of its slice for row / token l % 32 (the same
+// input-to-slot map for weights and tokens, which is all an MFMA needs).
+// The accumulation order is this kernel's own (fp32 MFMA sums over 16 inputs in order, splits in order): results agree with the
 // reference's cuBLAS route and with the oracle's dequantized weights times x in fp64 within fp32-accumulation error.
-#include <algorithm>
+#include <mutex>
 #include <type_traits>
 
 #include "agens_kernels.h"
@@ -39,6 +42,7 @@
 
 
 namespace agq {
+int num_cus();
 void* stream_scratch(hipStream_t s, size_t bytes);
 
 namespace {
@@ -46,9 +50,10 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // slabs of 64 inputs (one row / token of a slab: 128 B in LDS), two LDS stages
-constexpr int kSlab = 64, kRowBytes = kSlab * 2, kStages = 2;
+constexpr int kSlab = 64, kRowBytes = kSlab * 2;
 constexpr int kRsrcWord3 = 0x00020000;  // raw buffer resource, dword 3 (CDNA)
 
 // f(integral_constant<int, I>) for I = B .. E - 1, unrolled at compile time
@@ -74,33 +79,11 @@ __device__ __forceinline__ void lds_dma16(__amdgpu_buffer_rsrc_t r, uint8_t* dst
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voff, soff, 0, 0);
 }
 
-// Morton spreading of 2-bit / 1-bit fields into nibbles (as the repack's inverse)
-__device__ __forceinline__ uint32_t spread2(uint32_t v) {
-  v &= 0xFFFFu;
-  v = (v ^ (v << 8)) & 0x00FF00FFu;
-  v = (v ^ (v << 4)) & 0x0F0F0F0Fu;
-  v = (v ^ (v << 2)) & 0x33333333u;
-  return v;
-}
-__device__ __forceinline__ uint32_t spread1(uint32_t v) {
-  v &= 0xFFu;
-  v = (v ^ (v << 12)) & 0x000F000Fu;
-  v = (v ^ (v << 6)) & 0x03030303u;
-  v = (v ^ (v << 3)) & 0x11111111u;
-  return v;
-}
-
-// the chunk as 4 words of 8 stored codes n (nibble i of word u = input 8 u + i) and the code offset: q = n - OFF
-template <int BITS>
-__device__ __forceinline__ void chunk_codes(const ChunkRaw<BITS>& d, uint32_t (&n)[4]) {
-  if constexpr (BITS == 4) {
-    n[0] = d.w[0], n[1] = d.w[1], n[2] = d.w[2], n[3] = d.w[3];
-  } else if constexpr (BITS == 2) {
-    n[0] = spread2(d.w[0]), n[1] = spread2(d.w[0] >> 16), n[2] = spread2(d.w[1]), n[3] = spread2(d.w[1] >> 16);
-  } else {
-    n[0] = spread2(d.w[0]) | (spread1(d.w[2]) << 2), n[1] = spread2(d.w[0] >> 16) | (spread1(d.w[2] >> 8) << 2);
-    n[2] = spread2(d.w[1]) | (spread1(d.w[2] >> 16) << 2), n[3] = spread2(d.w[1] >> 16) | (spread1(d.w[2] >> 24) << 2);
-  }
+// the workgroup meets (LDS ordered, loads in flight stay in flight)
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // 8 codes (one word) -> 8 bf16 bf16_rn((n - OFF) * s): the product is exact in fp32 (an fma of two exact terms), the
@@ -159,372 +142,283 @@ __device__ __forceinline__ u32x4 dequant_half(const HalfCodes& c, float s, int s
   return u32x4{o[0], o[1], o[2], o[3]};
 }
 
-// R output rows x T tokens per workgroup (2 R threads: a thread pair per row), wave tiles of 64 rows x WT tokens,
-// loads of the weights RING - 1 slabs ahead and of the tokens XR - 1 slabs ahead (RING a multiple of XR); XM: the
-// XCD-contiguous tile order (below); DMA: the tokens are loaded straight into XR LDS stages of their own (buffer
-// loads into LDS), not through registers
-template <int BITS, int G, int R, int T, int RING, int XR, bool XM, bool DMA, bool SPLIT>
-__global__ void __launch_bounds__(2 * R, R == 128 ? 2 : 1) wq_gemm_kernel(const uint16_t* __restrict__ x, int m,
+// SPLIT: k is split across workgroups; an item's fp32 tile goes to part[item] as its waves hold it (sum_splits_kernel)
+template <int BITS, int G, int T, bool SPLIT>
+__global__ void __launch_bounds__(512, T == 64 ? 4 : 1) wq_gemm_kernel(const uint16_t* __restrict__ x, int m,
                                                               const uint8_t* __restrict__ wt,
                                                               const uint16_t* __restrict__ st,
                                                               uint16_t* __restrict__ y, int n, int ldy, int k,
-                                                              int nrow_tiles, int ntok_tiles, float* __restrict__ part) {
-  constexpr int kRows = R, kToks = T, kThreads = 2 * R, kRing = RING;
-  // LDS: DMA: two weight stages of R rows, then XR token stages of T tokens; else two stages of R rows + T tokens
-  constexpr int kStage = DMA ? R * kRowBytes : (R + T) * kRowBytes, kXBase = DMA ? 2 * kStage : R * kRowBytes;
-  constexpr int kXStage = DMA ? T * kRowBytes : kStage;
-  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+                                                              int nrow_tiles, int ntok_tiles, int nsplit,
+                                                              float* __restrict__ part) {
+  constexpr int R = 256, NJ = T / 64, XPW = T / 64;  // 32-token tiles per wave, 1 KB token blocks per wave and slab
+  constexpr int kWStage = R * kRowBytes, kXStage = T * kRowBytes, kXBase = 2 * kWStage;
   constexpr int OFF = BITS == 4 ? 8 : BITS == 3 ? 4 : 2;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // workgroup -> (row tile, token tile).  Workgroup b runs on XCD b % 8.  XM: the tiles in token-major order
-  // (tile = token tile x row tiles + row tile) cut into 8 contiguous runs, XCD x taking run x, so that each XCD's
-  // workgroups share one or two token tiles (T tokens x k inputs) through its L2 while the weights stream; else blocks
-  // of 8 row tiles x all token tiles with the token tiles of a row tile 8 workgroups apart (same XCD: they share the
-  // row tile's weights).
-  const int b = blockIdx.x;
-  int rt, tt;
-  if constexpr (XM) {
-    const int per = (nrow_tiles * ntok_tiles + 7) >> 3, tile = (b & 7) * per + (b >> 3);
-    tt = tile / nrow_tiles, rt = tile - tt * nrow_tiles;
-    if (tt >= ntok_tiles) return;
-  } else {
-    const int grp = b / (8 * ntok_tiles), in = b - grp * 8 * ntok_tiles;
-    rt = grp * 8 + (in & 7), tt = in >> 3;
-  }
-  const int o0 = rt * kRows, t0 = tt * kToks;
-  if (o0 >= n || t0 >= m) return;  // the last group of 8 row tiles may be partial
+  constexpr int REC = 128 * BITS, CB = BITS == 4 ? 16 : 8;
+  constexpr int kWLoads = BITS == 3 ? 3 : 2;  // weight and scale loads of a slab
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // workgroup b runs on XCD b % 8 and takes item (b % 8) x per + b / 8: split-major, then token-major tiles, cut into 8
+  // contiguous runs
+  const int tiles = nrow_tiles * ntok_tiles, items = tiles * nsplit, per = (items + 7) >> 3;
+  const int item = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+  if (((int)blockIdx.x >> 3) >= per || item >= items) return;
+  const int sp = SPLIT ? item / tiles : 0, tile = item - sp * tiles;
+  const int tt = tile / nrow_tiles, rt = tile - tt * nrow_tiles;
+  const int o0 = rt * R, t0 = tt * T;
+  const int sb = SPLIT ? (int)((long long)sp * (k / kSlab) / nsplit) : 0;
+  const int nslab = SPLIT ? (int)((long long)(sp + 1) * (k / kSlab) / nsplit) - sb : k / kSlab;
 
-  // Per slab (64 inputs): thread (row lr, half lj) loads lane chunk 2 sl + lj of row lr's KT record (W4 16 B, W3
-  // 8 + 4 B, W2 8 B) and its scale (rows past n load row n - 1: their results are not written); the inputs are 1024
-  // 16-byte chunks (token c / 8, chunk c % 8), thread tid loading chunks tid + j * kThreads (8 consecutive threads read
-  // one token's 128 bytes; tokens past m read token 0 and are written as zeros).  Loads are issued kRing - 1 slabs
-  // ahead and every load is unconditional (a slab past the end loads the last one again, never used): loads under a
-  // branch make the compiler's wait counts conservative at the join, which drains the pipeline.
-  constexpr int XPT = kToks * 8 / kThreads;  // input chunks per thread and slab
-  constexpr int REC = 128 * BITS, CB = BITS == 4 ? 16 : 8;  // record bytes; bytes of a lane chunk's (low) words
   const int lr = tid >> 1, lj = tid & 1;
   const int orow = o0 + lr < n ? o0 + lr : n - 1;
-  // split-K (part != nullptr): workgroup (.., blockIdx.y) takes slabs [sb, sb + nslab) of the k range and writes its
-  // fp32 tile to part[blockIdx.y][token][row] (row stride n); a second kernel adds the splits in order
-  const int sb = SPLIT ? (int)((long long)blockIdx.y * (k / kSlab) / gridDim.y) : 0;
-  const int nslab = SPLIT ? (int)((long long)(blockIdx.y + 1) * (k / kSlab) / gridDim.y) - sb : k / kSlab;
-  // buffer loads: a per-lane offset fixed for the whole loop plus a per-slab scalar offset (no address arithmetic on
-  // the vector unit in the loop); every buffer is below 2 GB (checked by the launcher)
   const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(wt), (short)0, 0x7FFFFFFF,
                                                                       kRsrcWord3);
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(st), (short)0, 0x7FFFFFFF,
                                                                       kRsrcWord3);
-  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), (short)0,
-                                                                      DMA ? m * k * 2 : 0x7FFFFFFF, kRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), (short)0, m * k * 2,
+                                                                      kRsrcWord3);
   const int vw = orow * REC + lj * CB, vh = orow * REC + 256 + lj * 4, vs = orow * (1024 / G) * 2;
-  // register path: chunk c = tid + j kThreads is (token c / 8, chunk c % 8), tokens past m read token 0.  DMA:
-  // instruction j of wave w fills the 1 KB block b = w + (kThreads / 64) j of the stage (tokens 8 b .. 8 b + 7, 128 B
-  // each), lane l writing bytes 16 l .. 16 l + 15, i.e. token 8 b + l / 8 at slot l % 8, which holds the token's chunk
-  // (l % 8) ^ ((token >> 1) & 7); one offset vx[0] for all j (+ j x the block step), tokens past m reading zeros
-  // through the buffer's range (m k 2 bytes)
-  int vx[DMA ? 1 : XPT];
-  if constexpr (DMA) {
-    const int tk = 8 * wave + (lane >> 3), q = (lane & 7) ^ ((tk >> 1) & 7);  // ((tk + 64 j) >> 1) & 7 is the same
-    vx[0] = ((t0 + tk) * k + 8 * q) * 2;
-  } else {
-#pragma unroll
-    for (int j = 0; j < XPT; ++j) {
-      const int c = tid + j * kThreads, tk = c >> 3;
-      vx[j] = ((t0 + tk < m ? t0 + tk : 0) * k + 8 * (c & 7)) * 2;
-    }
-  }
-  const bool full = t0 + kToks <= m;  // every token of the tile exists (no zero selection)
-  int xsel[XPT];                      // else: per chunk, whether its token exists
-#pragma unroll
-  for (int j = 0; j < XPT; ++j) xsel[j] = t0 + ((tid + j * kThreads) >> 3) < m;
+  const int tk = 8 * wave + (lane >> 3), vx = ((t0 + tk) * k + 8 * ((lane & 7) ^ ((tk >> 1) & 7))) * 2;
 
-  struct WSlab {
-    ChunkRaw<BITS> w;
-  };
-  struct XSlab {
-    u32x4 xv[XPT];
-  };
-  static_assert(RING % XR == 0, "the token ring must divide the weight ring");
-  WSlab rg[kRing];
-  XSlab rx_[DMA ? 1 : XR];
-  auto issue_w = [&](int sl, WSlab& d) __attribute__((always_inline)) {
-    const int t = (sb + sl) >> 4, s16 = (sb + sl) & 15;  // tile, slab within the tile
-    const int tb = t * n * REC;
+  ChunkRaw<BITS> rg[2];
+  auto issue_w = [&](int sl, ChunkRaw<BITS>& d) __attribute__((always_inline)) {
+    sl = sb + (sl < nslab ? sl : nslab - 1);
+    const int t = sl >> 4, s16 = sl & 15, tb = t * n * REC;
     if constexpr (BITS == 4) {
-      d.w.w = __builtin_amdgcn_raw_buffer_load_b128(rw, vw, tb + s16 * 32, 0);
+      d.w = __builtin_amdgcn_raw_buffer_load_b128(rw, vw, tb + s16 * 32, 0);
     } else {
       typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
       const u32x2 lo = __builtin_amdgcn_raw_buffer_load_b64(rw, vw, tb + s16 * 16, 0);
       const uint32_t hi = BITS == 3 ? __builtin_amdgcn_raw_buffer_load_b32(rw, vh, tb + s16 * 8, 0) : 0u;
-      d.w.w = u32x4{lo[0], lo[1], hi, 0u};
+      d.w = u32x4{lo[0], lo[1], hi, 0u};
     }
-    d.w.s = __builtin_amdgcn_raw_buffer_load_b16(rs, vs, (t * n * (1024 / G) + (G == 128 ? s16 >> 1 : s16)) * 2, 0);
+    d.s = __builtin_amdgcn_raw_buffer_load_b16(rs, vs, (t * n * (1024 / G) + (G == 128 ? s16 >> 1 : s16)) * 2, 0);
   };
-  auto issue_x = [&](int sl, XSlab& d) __attribute__((always_inline)) {
-#pragma unroll
-    for (int j = 0; j < XPT; ++j)
-      if constexpr (!DMA) d.xv[j] = __builtin_amdgcn_raw_buffer_load_b128(rx, vx[j], (sb + sl) * kSlab * 2, 0);
-  };
-  // DMA: slab sl's tokens into token stage xs (every wave its XPT blocks)
   auto dma_x = [&](int sl, int xs) __attribute__((always_inline)) {
+    sl = sb + (sl < nslab ? sl : nslab - 1);
 #pragma unroll
-    for (int j = 0; j < XPT; ++j)
-      lds_dma16(rx, lds + kXBase + xs * kXStage + (wave + (kThreads / 64) * j) * 1024,
-                vx[0] + j * (kThreads / 64) * 8 * k * 2, (sb + sl) * kSlab * 2);
+    for (int j = 0; j < XPW; ++j)
+      lds_dma16(rx, lds + kXBase + xs * kXStage + (wave + 8 * j) * 1024, vx + j * 64 * k * 2, sl * kSlab * 2);
   };
-  // (the zero selection of tokens past m happens here, at the write: selecting at the load would wait for the data)
-  auto put = [&](const WSlab& d, const XSlab& dx, int stage) __attribute__((always_inline)) {
-    uint8_t* base = lds + stage * kStage;
-    const float s = bf2f(d.w.s);
-    if constexpr (BITS == 4) {
-      uint32_t nw[4];
-      chunk_codes<BITS>(d.w, nw);
-#pragma unroll
-      for (int u = 0; u < 4; ++u) *reinterpret_cast<u32x4*>(base + swz(lr, 4 * lj + u)) = dequant8<OFF>(nw[u], s);
-    } else {
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const HalfCodes hc = half_codes<BITS>(d.w, h);
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub)
-          *reinterpret_cast<u32x4*>(base + swz(lr, 4 * lj + 2 * h + sub)) = dequant_half<OFF>(hc, s, sub);
-      }
-    }
-    if constexpr (DMA) return;
-    uint8_t* xb = lds + kXBase + stage * kXStage;
-    if (full) {
-#pragma unroll
-      for (int j = 0; j < XPT; ++j) {
-        const int c = tid + j * kThreads;
-        *reinterpret_cast<u32x4*>(xb + swz(c >> 3, c & 7)) = dx.xv[j];
-      }
-    } else {
-      const u32x4 z = {0u, 0u, 0u, 0u};
-#pragma unroll
-      for (int j = 0; j < XPT; ++j) {
-        const int c = tid + j * kThreads;
-        *reinterpret_cast<u32x4*>(xb + swz(c >> 3, c & 7)) = xsel[j] ? dx.xv[j] : z;
-      }
-    }
+  // word u (8 inputs) of the thread's chunk, dequantized into weight stage `stage`
+  auto put = [&](const ChunkRaw<BITS>& d, int u, int stage) __attribute__((always_inline)) {
+    uint8_t* dst = lds + stage * kWStage + swz(lr, 4 * lj + u);
+    const float sc = bf2f(d.s);
+    if constexpr (BITS == 4)
+      *reinterpret_cast<u32x4*>(dst) = dequant8<OFF>(d.w[u], sc);
+    else
+      *reinterpret_cast<u32x4*>(dst) = dequant_half<OFF>(half_codes<BITS>(d, u >> 1), sc, u & 1);
   };
 
-  // wave tiles of 64 rows x WT tokens
-  constexpr int RW = kRows / 64, WT = kToks / (kThreads / 64 / RW), NJ = WT / 16;  // waves along the rows
-  const int wr = (wave % RW) * 64, wtk = (wave / RW) * WT;
-  const int lrow = lane & 15, lsub = lane >> 4;
-  f32x4 acc[4][NJ];
+  const int wr = (wave & 3) * 64, wtk = (wave >> 2) * (T / 2);
+  const int l32 = lane & 31, hi = lane >> 5;
+  f32x16 acc[2][NJ];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  auto compute = [&](int stage, int xs) __attribute__((always_inline)) {
-    const uint8_t* A = lds + stage * kStage;
-    const uint8_t* B = lds + kXBase + xs * kXStage;
+    for (int j = 0; j < NJ; ++j)
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {  // 32-input slices of the slab
-      const int q = 4 * h + lsub;
-      bf16x8 av[4], bv[NJ];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) av[i] = *reinterpret_cast<const bf16x8*>(A + swz(wr + 16 * i + lrow, q));
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) bv[j] = *reinterpret_cast<const bf16x8*>(B + swz(wtk + 16 * j + lrow, q));
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i], bv[j], acc[i][j], 0, 0, 0);
-    }
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  struct Frag {
+    bf16x8 a[2], b[NJ];
   };
-
-  // compute(stage, xs) with put's weight half interleaved (DMA path): after each 16 MFMAs one of the next slab's four
-  // words is dequantized and written, the MFMAs and that VALU work alternating in each region (a wave issues in
-  // order, so VALU work placed between its MFMAs runs while they do)
-  auto compute_put = [&](int stage, int xs, const WSlab& d, int wstage) __attribute__((always_inline)) {
-    const uint8_t* A = lds + stage * kStage;
-    const uint8_t* B = lds + kXBase + xs * kXStage;
-    uint8_t* base = lds + wstage * kStage;
-    uint32_t nw[4];
-    if constexpr (BITS == 4) chunk_codes<BITS>(d.w, nw);
-    const float sc = bf2f(d.w.s);
+  auto frag = [&](int stage, int s, Frag& f) __attribute__((always_inline)) {
+    const int q = 2 * s + hi;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int q = 4 * h + lsub;
-      HalfCodes hc;
-      if constexpr (BITS != 4) hc = half_codes<BITS>(d.w, h);
-      bf16x8 av[4], bv[NJ];
+    for (int i = 0; i < 2; ++i)
+      f.a[i] = *reinterpret_cast<const bf16x8*>(lds + stage * kWStage + swz(wr + 32 * i + l32, q));
 #pragma unroll
-      for (int i = 0; i < 4; ++i) av[i] = *reinterpret_cast<const bf16x8*>(A + swz(wr + 16 * i + lrow, q));
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) bv[j] = *reinterpret_cast<const bf16x8*>(B + swz(wtk + 16 * j + lrow, q));
-      // W4: the slice's MFMA run at raised wave priority, so that the SIMD's other wave, in its dequantization or
-      // operand reads, yields issue slots to it (measured: W4 8-10 % faster; W3, whose unpacking is heavier, slower)
-      if constexpr (BITS == 4) __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-      for (int ih = 0; ih < 2; ++ih) {
-#pragma unroll
-        for (int i = 2 * ih; i < 2 * ih + 2; ++i)
-#pragma unroll
-          for (int j = 0; j < NJ; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i], bv[j], acc[i][j], 0, 0, 0);
-        const int u = 2 * h + ih;
-        if constexpr (BITS == 4)
-          *reinterpret_cast<u32x4*>(base + swz(lr, 4 * lj + u)) = dequant8<OFF>(nw[u], sc);
-        else
-          *reinterpret_cast<u32x4*>(base + swz(lr, 4 * lj + u)) = dequant_half<OFF>(hc, sc, ih);
-        static_for<0, 2 * NJ>([&](auto) __attribute__((always_inline)) {
-          __builtin_amdgcn_sched_group_barrier(0x0008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x0002, 3, 0);  // 1 MFMA, 3 VALU
-        });
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if constexpr (BITS == 4) __builtin_amdgcn_s_setprio(0);
-    }
+    for (int j = 0; j < NJ; ++j)
+      f.b[j] = *reinterpret_cast<const bf16x8*>(lds + kXBase + stage * kXStage + swz(wtk + 32 * j + l32, q));
   };
-
-  // Pipeline over slabs: two LDS stages, kRing weight register sets and XR token register sets.  Iteration sl:
-  // barrier (slab sl in LDS; every wave done with slab sl - 1), issue the token loads of slab sl + XR - 1 and then the
-  // weight loads of slab sl + kRing - 1 (in this order: the loads' counter is in order, and the tokens, read from L2,
-  // are needed first), compute slab sl from its stage, write slab sl + 1 (dequantized) into the other stage.
-  constexpr int D = kRing - 1, DX = XR - 1;
-  if constexpr (DMA) {
-    // Iteration sl: wait for all of this wave's loads (its token DMA of slab sl among them; the weight loads still
-    // outstanding were issued a slab earlier, so this costs little, and it holds whatever order the loads were issued
-    // in), barrier (every wave's DMA of slab sl landed; every wave done with slab sl - 1), DMA of slab sl + DX into
-    // the token stage slab sl - 1 used, weight loads of slab sl + D, compute slab sl, write slab sl + 1's weights
-    // (dequantized) into the other weight stage.
-    static_assert(DX >= 1, "token DMA pipeline");
-    constexpr int kVmcnt0 = 0x0F70;  // s_waitcnt immediate: vector memory counter 0, the others unconstrained
+  auto mfma = [&](const Frag& f) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < DX; ++i) dma_x(i < nslab ? i : nslab - 1, i);
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int i = 0; i < D; ++i) issue_w(i < nslab ? i : nslab - 1, rg[i]);
-    put(rg[0], rx_[0], 0);
-    auto iter = [&](int sl, auto S, bool last_ok) __attribute__((always_inline)) {
-      constexpr int r1 = (decltype(S)::value + 1) % kRing, rd = (decltype(S)::value + D) % kRing;
-      constexpr int xc = decltype(S)::value % XR, xd = (decltype(S)::value + DX) % XR;
-      __builtin_amdgcn_s_waitcnt(kVmcnt0);
-      __syncthreads();
-      dma_x(sl + DX < nslab ? sl + DX : nslab - 1, xd);
-      issue_w(sl + D < nslab ? sl + D : nslab - 1, rg[rd]);
-      if (last_ok) {
-        compute_put(sl & 1, xc, rg[r1], (sl + 1) & 1);
-      } else {
-        compute(sl & 1, xc);
-        if (sl + 1 < nslab) put(rg[r1], rx_[0], (sl + 1) & 1);
-      }
-    };
-    int sl = 0;
-    for (; sl + kRing < nslab; sl += kRing)  // every iteration here has a next slab
-      static_for<0, kRing>([&](auto I) __attribute__((always_inline)) { iter(sl + decltype(I)::value, I, true); });
-    static_for<0, kRing>([&](auto I) __attribute__((always_inline)) {
-      if (sl + decltype(I)::value < nslab) iter(sl + decltype(I)::value, I, false);
+      for (int j = 0; j < NJ; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[i], f.b[j], acc[i][j], 0, 0, 0);
+  };
+  // the slice's MFMAs and its other instructions in turn: one MFMA, NV VALU
+  auto mix = [&](auto NV) __attribute__((always_inline)) {
+    static_for<0, 2 * NJ>([&](auto) __attribute__((always_inline)) {
+      __builtin_amdgcn_sched_group_barrier(0x0008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x0002, decltype(NV)::value, 0);
     });
-  } else {
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  constexpr int kVmcnt0 = 0x0F70;  // s_waitcnt immediate: vector memory counter 0, the others unconstrained
+  constexpr int kVmcntW = kVmcnt0 | kWLoads;  // at most one slab's weight loads outstanding
+  Frag f0, f1;
+  issue_w(0, rg[0]);
+  issue_w(1, rg[1]);
+  dma_x(0, 0);
 #pragma unroll
-    for (int i = 0; i < DX; ++i) issue_x(i < nslab ? i : nslab - 1, rx_[i]);
-#pragma unroll
-    for (int i = 0; i < D; ++i) issue_w(i < nslab ? i : nslab - 1, rg[i]);
-    put(rg[0], rx_[0], 0);
-    auto iter = [&](int sl, auto S) __attribute__((always_inline)) {
-      constexpr int r1 = (decltype(S)::value + 1) % kRing, rd = (decltype(S)::value + D) % kRing;
-      constexpr int x1 = (decltype(S)::value + 1) % XR, xd = (decltype(S)::value + DX) % XR;
-      __syncthreads();
-      if constexpr (DX > 0) issue_x(sl + DX < nslab ? sl + DX : nslab - 1, rx_[xd]);
-      issue_w(sl + D < nslab ? sl + D : nslab - 1, rg[rd]);
-      compute(sl & 1, sl & 1);
-      if constexpr (DX == 0) issue_x(sl + 1 < nslab ? sl + 1 : nslab - 1, rx_[x1]);
-      if (sl + 1 < nslab) put(rg[r1], rx_[x1], (sl + 1) & 1);
-    };
-    int sl = 0;
-    for (; sl + kRing <= nslab; sl += kRing)
-      static_for<0, kRing>([&](auto I) __attribute__((always_inline)) { iter(sl + decltype(I)::value, I); });
-    static_for<0, kRing - 1>([&](auto I) __attribute__((always_inline)) {
-      if (sl + decltype(I)::value < nslab) iter(sl + decltype(I)::value, I);
-    });
+  for (int u = 0; u < 4; ++u) put(rg[0], u, 0);
+  __builtin_amdgcn_s_waitcnt(kVmcnt0);
+  lds_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  dma_x(1, 1);
+  __builtin_amdgcn_sched_barrier(0);
+  issue_w(2, rg[0]);
+  __builtin_amdgcn_sched_barrier(0);
+  frag(0, 0, f0);
+  // slab sl in stage S; f0 holds its first slice.  The order of the token and weight loads is pinned (the counted wait
+  // above relies on it); loads past the last slab read it again and are not used
+  auto body = [&](int sl, auto S) __attribute__((always_inline)) {
+    constexpr int s = decltype(S)::value;
+    ChunkRaw<BITS>& d = rg[s ^ 1];  // slab sl + 1
+    frag(s, 1, f1);
+    mfma(f0);
+    put(d, 0, s ^ 1);
+    mix(std::integral_constant<int, 4>());
+    frag(s, 2, f0);
+    mfma(f1);
+    put(d, 1, s ^ 1);
+    put(d, 2, s ^ 1);
+    mix(std::integral_constant<int, 7>());
+    frag(s, 3, f1);
+    mfma(f0);
+    put(d, 3, s ^ 1);
+    mix(std::integral_constant<int, 4>());
+    // the next slab's token loads have landed (issued a slab ago, before that slab's weight loads)
+    __builtin_amdgcn_s_waitcnt(kVmcntW);
+    lds_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    dma_x(sl + 2, s);
+    __builtin_amdgcn_sched_barrier(0);
+    issue_w(sl + 3, d);
+    __builtin_amdgcn_sched_barrier(0);
+    frag(s ^ 1, 0, f0);
+    mfma(f1);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  int sl = 0;
+  for (; sl + 1 < nslab; sl += 2) {
+    body(sl, std::integral_constant<int, 0>());
+    body(sl + 1, std::integral_constant<int, 1>());
   }
+  if (sl < nslab) body(sl, std::integral_constant<int, 0>());
+  __builtin_amdgcn_s_waitcnt(kVmcnt0);  // no load into LDS outlives the workgroup
 
-  // D: lane holds rows 4 (lane / 16) + e of its 16-row tile for token lane % 16
+  // 4 rows of a lane's output in one 8-byte store where the rows stay aligned
+  const bool vec = ((n | ldy) & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 7) == 0;
+  // D: register 4 g + e of lane l holds row 8 g + 4 (l / 32) + e of its 32-row tile for token l % 32
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    const int t = t0 + wtk + 16 * j + lrow;
+    const int t = t0 + wtk + 32 * j + l32;
     if (t >= m) continue;
-    if (SPLIT) {  // the fp32 tile
-      float* pr = part + ((size_t)blockIdx.y * m + t) * n;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r0 = o0 + wr + 16 * i + 4 * lsub;
-        if ((n & 3) == 0 && r0 < n) {
-          *reinterpret_cast<f32x4*>(pr + r0) = acc[i][j];
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int r0 = o0 + wr + 32 * i + 8 * g + 4 * hi;
+        if constexpr (SPLIT) {
+          reinterpret_cast<f32x4*>(part)[((size_t)item * (64 * NJ) + ((wave * NJ + j) * 2 + i) * 4 + g) * 64 + lane] =
+              f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
         } else {
+          uint16_t* yr = y + (size_t)t * ldy;
+          const bf16x2 lo = {(__bf16)acc[i][j][4 * g], (__bf16)acc[i][j][4 * g + 1]};
+          const bf16x2 up = {(__bf16)acc[i][j][4 * g + 2], (__bf16)acc[i][j][4 * g + 3]};
+          if (vec) {
+            if (r0 < n)
+              *reinterpret_cast<uint2*>(yr + r0) =
+                  make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, up));
+          } else {
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (r0 + e < n) pr[r0 + e] = acc[i][j][e];
+            for (int e = 0; e < 4; ++e)
+              if (r0 + e < n) yr[r0 + e] = __builtin_bit_cast(uint16_t, (__bf16)acc[i][j][4 * g + e]);
+          }
         }
       }
-      continue;
-    }
-    uint16_t* yr = y + (size_t)t * ldy;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r0 = o0 + wr + 16 * i + 4 * lsub;
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (r0 + e < n) yr[r0 + e] = __builtin_bit_cast(uint16_t, (__bf16)acc[i][j][e]);
-    }
   }
 }
 
-// y[t][o] = bf16(part[0][t][o] + part[1][t][o] + ... + part[S - 1][t][o]), the splits in order; 4 rows per thread
-__global__ void __launch_bounds__(256) sum_splits_kernel(const float* __restrict__ part, int nsplit, int m, int n,
-                                                         uint16_t* __restrict__ y, int ldy) {
-  const int n4 = (n + 3) >> 2;
-  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (long long)m * n4) return;
-  const int t = (int)(i / n4), o = (int)(i - (long long)t * n4) * 4;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  if ((n & 3) == 0) {  // 16-byte partial loads, one 8-byte store
-    for (int sp = 0; sp < nsplit; ++sp) {
-      const f32x4 v = *reinterpret_cast<const f32x4*>(part + ((size_t)sp * m + t) * n + o);
+// y = bf16 of the splits' partials added in order.  A split's partials of a tile lie as its waves hold them (16 bytes per
+// lane: 4 rows of one token; 64 NJ such kilobytes per tile), so that they are written and read in whole lines; a thread
+// sums one 16-byte piece.  Eight splits' loads are requested before their sums (splits past the last one read the last
+// one again and are not added): one memory round trip per eight splits instead of one per split.
+__global__ void __launch_bounds__(256) sum_splits_kernel(const f32x4* __restrict__ part, int nsplit, int m, int n,
+                                                         uint16_t* __restrict__ y, int ldy, int nrow_tiles, int tiles,
+                                                         int nj) {
+  const int f = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;  // kilobyte of the tile, its lane
+  const int tile = blockIdx.y, tt = tile / nrow_tiles, rt = tile - tt * nrow_tiles;
+  const int wj = f >> 3, wave = wj / nj, j = wj - wave * nj;
+  const int t = (tt * 2 + (wave >> 2)) * 32 * nj + 32 * j + (lane & 31);
+  const int o = rt * 256 + (wave & 3) * 64 + 8 * (f & 7) + 4 * (lane >> 5);
+  if (t >= m || o >= n) return;
+  const f32x4* p = part + ((size_t)tile * (64 * nj) + f) * 64 + lane;
+  const size_t step = (size_t)tiles * (64 * nj) * 64;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < nsplit; s0 += 8) {
+    f32x4 v[8];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[e] += v[e];
-    }
-    const bf16x2 lo = {(__bf16)acc[0], (__bf16)acc[1]}, hi = {(__bf16)acc[2], (__bf16)acc[3]};
-    uint16_t* yo = y + (size_t)t * ldy + o;
-    if ((ldy & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 7) == 0) {  // 8-byte aligned (y may be a column offset)
-      *reinterpret_cast<uint2*>(yo) = make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
-    } else {
+    for (int i = 0; i < 8; ++i) v[i] = p[(s0 + i < nsplit ? s0 + i : nsplit - 1) * step];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) yo[e] = __builtin_bit_cast(uint16_t, (__bf16)acc[e]);
-    }
-    return;
+    for (int i = 0; i < 8; ++i)
+      if (s0 + i < nsplit) acc += v[i];
   }
-  for (int sp = 0; sp < nsplit; ++sp) {
-    const float* pr = part + ((size_t)sp * m + t) * n + o;
+  const bf16x2 lo = {(__bf16)acc[0], (__bf16)acc[1]}, hi = {(__bf16)acc[2], (__bf16)acc[3]};
+  uint16_t* yo = y + (size_t)t * ldy + o;
+  if (o + 4 <= n && (ldy & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 7) == 0) {  // y may be a column offset
+    *reinterpret_cast<uint2*>(yo) = make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
+  } else {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      if (o + e < n) acc[e] += pr[e];
+      if (o + e < n) yo[e] = __builtin_bit_cast(uint16_t, (__bf16)acc[e]);
   }
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-    if (o + e < n) y[(size_t)t * ldy + o + e] = __builtin_bit_cast(uint16_t, (__bf16)acc[e]);
 }
 
-template <int BITS, int G, int R, int T, int RING, int XR, bool XM, bool DMA, bool SPLIT = false>
+template <int BITS, int G, int T, bool SPLIT>
 int launch_tiles(const void* x, int m, const void* wt, const void* st, void* y, int n, int ldy, int k, hipStream_t s,
-                 int nsplit = 1, float* part = nullptr) {
-  const int nrt = (n + R - 1) / R, ntt = (m + T - 1) / T;
-  const long long grid = XM ? ((long long)nrt * ntt + 7) / 8 * 8 : (long long)((nrt + 7) / 8) * 8 * ntt;
+                int nsplit = 1, float* part = nullptr) {
+  const int nrt = (n + 255) / 256, ntt = (m + T - 1) / T;
+  const long long grid = ((long long)nrt * ntt * nsplit + 7) / 8 * 8;
   if (grid > 0x7FFFFFFF) return AK_INVALID;
-  hipLaunchKernelGGL((wq_gemm_kernel<BITS, G, R, T, RING, XR, XM, DMA, SPLIT>), dim3((unsigned)grid, (unsigned)nsplit), dim3(2 * R),
-                     DMA ? (2 * R + XR * T) * kRowBytes : kStages * (R + T) * kRowBytes, s, static_cast<const uint16_t*>(x), m,
+  hipLaunchKernelGGL((wq_gemm_kernel<BITS, G, T, SPLIT>), dim3((unsigned)grid), dim3(512),
+                     2 * (256 + T) * kRowBytes, s, static_cast<const uint16_t*>(x), m,
                      static_cast<const uint8_t*>(wt), static_cast<const uint16_t*>(st), static_cast<uint16_t*>(y), n,
-                     ldy, k, nrt, ntt, part);
-  if (nsplit > 1) {
-    const long long items = (long long)m * ((n + 3) / 4);
-    hipLaunchKernelGGL(sum_splits_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s, part, nsplit, m, n,
-                       static_cast<uint16_t*>(y), ldy);
-  }
+                     ldy, k, nrt, ntt, nsplit, part);
+  if (SPLIT)
+    hipLaunchKernelGGL(sum_splits_kernel, dim3(T / 4, (unsigned)(nrt * ntt)), dim3(256), 0, s,
+                       reinterpret_cast<const f32x4*>(part), nsplit, m, n, static_cast<uint16_t*>(y), ldy, nrt,
+                       nrt * ntt, T / 64);
   return (int)hipGetLastError();
+}
+
+// The tiling of a launch: T tokens per tile and the number of k splits, by the estimated time
+//   rounds x (slabs x slab time(T) + 3) + (split: 4 + the fp32 partials written and read at 8 TB/s) us,
+// rounds = workgroups per XCD / CUs per XCD, rounded up (one workgroup per CU at a time: at T = 64 two fit, but share
+// the same throughput).  Slab times measured at 240 workgroups (us): 0.78 at 64 tokens, 1.12 at 128, 1.42 at 192, 1.75 at
+// 256 (the dequantization and the weight tile's LDS traffic do not shrink with T).  So wide linears take the largest
+// tile that does not pad too many tokens, and narrow or short ones split k until one round is nearly full.  Measured
+// (us, T x splits): down 5120 x 27648 W2 at 333 tokens 192 x 6 112, 128 x 4 126, 256 x 6 130; at 256 tokens 128 x 6 91,
+// 128 x 8 119 (a second round); at 64 tokens 64 x 12 40, 64 x 8 49, 64 x 16 46; o 5120 x 5120 W4 at 256 tokens
+// 128 x 6 30, 128 x 4 34, 128 x 8 39.
+struct Tiling {
+  int T, split;
+};
+Tiling pick_tiling(int m, int n, int nslab, bool may_split) {
+  const int xcd_cus = num_cus() / 8 > 0 ? num_cus() / 8 : 1;
+  Tiling best = {256, 1};
+  double best_us = 1e30;
+  for (int T = 64; T <= 256; T += 64) {
+    const double slab = T == 256 ? 1.75 : T == 192 ? 1.42 : T == 128 ? 1.12 : 0.78;
+    const long long tiles = (long long)((n + 255) / 256) * ((m + T - 1) / T);
+    for (int sp = 1; sp <= (may_split ? 32 : 1) && (sp == 1 || nslab / sp >= 4); ++sp) {
+      const long long items = tiles * sp, rounds = ((items + 7) / 8 + xcd_cus - 1) / xcd_cus;
+      const double us = (double)rounds * ((nslab + sp - 1) / sp * slab + 3.0) +
+                        (sp > 1 ? 4.0 + 2048.0 * (double)items * T / 8e6 : 0.0);
+      if (us < best_us) best_us = us, best = {T, sp};
+    }
+  }
+  return best;
+}
+
+template <int BITS, int G, int T>
+int launch_t(const void* x, int m, const void* wt, const void* st, void* y, int n, int ldy, int k, hipStream_t s,
+             int nsplit, float* part) {
+  return part ? launch_tiles<BITS, G, T, true>(x, m, wt, st, y, n, ldy, k, s, nsplit, part)
+              : launch_tiles<BITS, G, T, false>(x, m, wt, st, y, n, ldy, k, s);
 }
 
 template <int BITS, int G>
@@ -532,29 +426,25 @@ int launch_gemm(const void* x, int m, const void* wt, const void* st, void* y, i
   // 32-bit buffer offsets: the weights, scales and inputs must each stay below 2 GB
   if ((long long)kpad(k) / 1024 * n * 128 * BITS >= (1ll << 31) || (long long)m * k * 2 >= (1ll << 31))
     return AK_INVALID;
-  // 256 x 256 tiles above 128 tokens where there are enough of them to fill the GPU (measured: from about 160 tiles
-  // on, e.g. gate_up 55296 rows from 129 tokens, the 5120-row linears from 2048), else 128 x 128 tiles at two
-  // workgroups per CU
-  const long long big_tiles = (long long)((n + 255) / 256) * ((m + 255) / 256);
-  // (the weights 3 slabs ahead for W4 / W2, 1 for W3: a deeper ring spills W3's registers, measured 10 % slower; W4 /
-  // W2 are 5-11 % slower with 1)
-  if (m > 128 && big_tiles >= 160)
-    return launch_tiles<BITS, G, 256, 256, BITS == 3 ? 2 : 4, 2, true, true>(x, m, wt, st, y, n, ldy, k, s);
-  // 128 x 128 tiles; where there are fewer than 384 (measured: below that, splitting k wins over the partials'
-  // extra traffic), k is split across workgroups up to 512 of them (at least 8 slabs per split): fp32 partial tiles in
-  // the stream's scratch after its first 4 KB (the GEMV kernels' row-range counters, which stay zero between
-  // launches), summed in order by a second kernel; one pass where the scratch is not available (e.g. first use under
+  // fp32 partial tiles of a split launch: in the stream's scratch after its first 4 KB (the GEMV kernels' row-range
+  // counters, which stay zero between launches); one pass where the scratch is not available (e.g. first use under
   // stream capture)
-  const long long tiles = (long long)((n + 127) / 128) * ((m + 127) / 128);
-  int nsplit = 1;
-  if (tiles < 384) nsplit = (int)std::min<long long>((512 + tiles - 1) / tiles, std::min(64, k / kSlab / 8));
+  Tiling tl = pick_tiling(m, n, k / kSlab, true);
   float* part = nullptr;
-  if (nsplit > 1) {
-    if (void* z = stream_scratch(s, 4096 + (size_t)nsplit * m * n * 4))
+  std::unique_lock<std::mutex> lock;
+  if (tl.split > 1) {
+    lock = std::unique_lock<std::mutex>(scratch_mutex(s));  // the two kernels of a split launch stay together
+    if (void* z = stream_scratch(s, 4096 + (size_t)tl.split * ((n + 255) / 256) * ((m + tl.T - 1) / tl.T) * 1024 * tl.T))
       part = reinterpret_cast<float*>(static_cast<uint8_t*>(z) + 4096);
+    else
+      tl = pick_tiling(m, n, k / kSlab, false);
   }
-  if (part) return launch_tiles<BITS, G, 128, 128, 4, 4, false, false, true>(x, m, wt, st, y, n, ldy, k, s, nsplit, part);
-  return launch_tiles<BITS, G, 128, 128, 4, 4, false, false>(x, m, wt, st, y, n, ldy, k, s);
+  switch (tl.T) {
+    case 64: return launch_t<BITS, G, 64>(x, m, wt, st, y, n, ldy, k, s, tl.split, part);
+    case 128: return launch_t<BITS, G, 128>(x, m, wt, st, y, n, ldy, k, s, tl.split, part);
+    case 192: return launch_t<BITS, G, 192>(x, m, wt, st, y, n, ldy, k, s, tl.split, part);
+    default: return launch_t<BITS, G, 256>(x, m, wt, st, y, n, ldy, k, s, tl.split, part);
+  }
 }
 
 }  // namespace

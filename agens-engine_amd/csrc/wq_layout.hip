@@ -38,6 +38,11 @@ ScratchOverride& scratch_override() {
   return o;
 }
 
+std::mutex& scratch_mutex(hipStream_t s) {
+  static std::mutex m[64];  // streams share one only by chance of their address
+  return m[(reinterpret_cast<uintptr_t>(s) >> 6) & 63];
+}
+
 void* stream_scratch(hipStream_t s, size_t bytes) {
   const ScratchOverride& o = scratch_override();
   if (o.on) return bytes <= o.bytes ? o.p : nullptr;

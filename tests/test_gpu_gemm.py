@@ -149,6 +149,26 @@ def test_gemm_wide_tiles_exact_on_small_integer_operands(bits):
     assert (y[:, n:] == 0x7FC1).all()
 
 
+# every tile width (64, 128, 192, 256 tokens) at its edges, with few and odd numbers of 64-input slabs (the pipeline's
+# start and end), in one round of unsplit tiles (157 row tiles) and with k split across workgroups (1 to 20 row tiles)
+@pytest.mark.parametrize("bits,group,m,n,k", [
+    (4, 128, 64, 40001, 128), (3, 64, 65, 40001, 64), (2, 64, 128, 40001, 192), (3, 128, 129, 40000, 256),
+    (4, 64, 192, 40001, 64), (2, 128, 193, 40000, 384), (3, 64, 256, 40001, 192),
+    (2, 128, 1, 257, 2304), (4, 64, 64, 255, 1088), (3, 128, 65, 1, 4096), (4, 128, 129, 5120, 1152),
+    (2, 64, 200, 2331, 2752), (3, 128, 333, 5117, 2304), (4, 128, 512, 2050, 1024)])
+def test_gemm_tilings_exact_on_small_integer_operands(bits, group, m, n, k):
+    """Integer inputs and power-of-two scales: every product and partial sum is exact in fp32 (|sum| < 2^24 units of the
+    smallest scale), so every output must equal the fp64 product rounded once to bf16."""
+    L = make(8750 + bits + m, n, k, group, bits, scale_pow2=True)
+    rng = np.random.default_rng(8751 + m)
+    x = f2bf_array(rng.integers(-3, 4, (m, k)).astype(np.float32))
+    ld = n + 3
+    y = gemm(L, Dev.of(x), m, ldy=ld, fill=0x7FC1)
+    ref = bf2f_array(x).astype(np.float64) @ bf2f_array(dequant_host(L)).astype(np.float64).T
+    assert np.array_equal(y[:, :n], f2bf_array(ref.astype(np.float32)))
+    assert (y[:, n:] == 0x7FC1).all()
+
+
 def test_split_k_gemm_leaves_gemv_scratch_intact():
     """A narrow long-k GEMM splits k across workgroups (fp32 partials in the stream's scratch); the split-K GEMV
     launches on the same stream keep their row-range counters in the first 4 KB of that scratch, zero between
