@@ -6,115 +6,204 @@
 // same for every m).  The reference's bits come from its MMA instruction's internal accumulation, which no other
 // hardware reproduces; this kernel keeps the reference's contract instead -- fp32 accumulation, the bias added in fp32
 // before the one bf16 rounding, and an order that does not depend on m:
-//   - a workgroup owns 16 rows; its 8 waves take the 64-input k-steps s = w, w + 8, w + 16, ... (wave w; four steps'
-//     loads issued at a time), each step two
-//     v_mfma_f32_16x16x32_bf16 (inputs [64 s, 64 s + 32) then [64 s + 32, 64 s + 64)) accumulating in fp32;
+//   - k is cut into 64-input steps and those into 8 contiguous chunks, chunk p = steps [p S / 8, (p + 1) S / 8) of S;
+//     wave p of a workgroup takes chunk p for the workgroup's 16 RB rows, each step two v_mfma_f32_16x16x32_bf16 (inputs
+//     [64 s, 64 s + 32) then [64 s + 32, 64 s + 64)) accumulating in fp32;
 //   - the MFMA's A operand is 16 weight rows, its B operand 16 tokens: the columns of the result are independent, so a
 //     token's sums do not depend on the other tokens; more than 16 tokens are more B tiles of the same steps;
-//   - the 8 waves' partial sums are added in wave order (from wave 0), then the bias, then the bf16 rounding.
-// Operand layout: lane l holds inputs 8 (l / 16) .. + 8 of row (A) / token (B) l % 16 of the 32-input slice (one 16-byte
-// load each); any input-to-slot map gives the same sum as long as A and B use the same one.  D: lane l holds rows
-// 4 (l / 16) + i, i < 4, of token l % 16.
+//   - the 8 chunks' partial sums are added in order (from chunk 0), then the bias, then the bf16 rounding.
+// Operands: lane (c, h) = (l % 16, l / 16) holds inputs 8 h .. + 8 of row (A) / token (B) c of the 32-input slice; any
+// input-to-slot map gives the same sum as long as A and B use the same one.  D: lane (c, h) holds rows 4 h + i, i < 4, of
+// token c.
+// What bounds it: at few tokens the HBM stream and the latency of a short chain (5120 x 5120: 10 steps per wave), at
+// more the activations, which every workgroup reads whole from L2.  So every load instruction reads whole 128-byte
+// lines of 8 rows (or tokens): the lanes of a pair load the two halves of one row's line and swap them by DPP (own_row);
+// the next KU steps are requested before these are used; rows past n, tokens past m and steps past a chunk read zeros
+// through the buffers' range, which costs no memory traffic; and a workgroup takes 32 rows where that saves a round of
+// workgroups or activation traffic (rows_per_workgroup).  Measured (us, before = half-line loads at clamped addresses,
+// one row block per workgroup): 5120 x 5120 at 1 / 16 / 64 / 128 tokens 20.4 / 28.6 / 54.7 / 89.9 -> 13.2 / 15.8 / 27.5 /
+// 40.4; 8000 x 8192 at 4 tokens 35.0 -> 22.0 (5.95 TB/s).  16 waves per workgroup were slower (5120 x 5120 at 1 token
+// 18.5), and so were 3 or 4 steps per request group (19.7, 18.0 at 16 tokens).
 #include "agens_kernels.h"
 #include "wq_common.h"
 
+#include <algorithm>
+
 namespace agq {
+
+int num_cus();
+
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-constexpr int kWaves = 8;
+constexpr int NW = 8;  // waves per workgroup, chunks of k
+constexpr int kRsrcWord3 = 0x00020000;  // raw buffer resource, dword 3 (CDNA)
 
-__device__ __forceinline__ bf16x8 as_bf16x8(const uint4 v) {
-  bf16x8 r;
-  __builtin_memcpy(&r, &v, 16);
-  return r;
+// a = load 0, b = load 1 of a lane pair (lanes 2 i, 2 i + 1: row 2 i, then row 2 i + 1; the even lane the first half of
+// the line, the odd lane the second) -> the first and second half of the lane's own row
+__device__ __forceinline__ void own_row(u32x4& a, u32x4& b, bool odd) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t v = odd ? a[i] : b[i];  // what the partner lane needs
+    const uint32_t r = (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true);  // quad_perm [1, 0, 3, 2]
+    a[i] = odd ? r : a[i];
+    b[i] = odd ? b[i] : r;
+  }
 }
 
-// TT token tiles of 16 per launch (tokens [0, 16 TT) of x; m <= 16 TT)
-template <int TT>
-__global__ void __launch_bounds__(kWaves * 64) bi_gemv_kernel(const uint16_t* __restrict__ x, int m,
+// TT token tiles of 16 (m <= 16 TT), RB row blocks of 16 per workgroup, KU steps per group of requests
+template <int TT, int RB, int KU>
+__global__ void __launch_bounds__(NW * 64) bi_gemv_kernel(const uint16_t* __restrict__ x, int m,
                                                               const uint16_t* __restrict__ w,
                                                               const uint16_t* __restrict__ bias,
                                                               uint16_t* __restrict__ y, int n, int k, long ldy) {
-  __shared__ f32x4 red[kWaves][TT][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = (int)blockIdx.x * 16 + (lane & 15);  // this lane's A row
-  const int kq = 8 * (lane >> 4);                      // its inputs within a 32-input slice
-  const bool rok = r < n;
-  const uint16_t* wr = w + (size_t)(rok ? r : 0) * k + kq;
-  f32x4 acc[TT];
+  extern __shared__ f32x4 red[];  // [NW][RB * TT][64]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, h = lane >> 4;
+  const bool odd = c & 1;
+  const int row0 = (int)blockIdx.x * 16 * RB;
+  const int steps = (k + 63) >> 6, s_lo = wave * steps / NW, s_hi = (wave + 1) * steps / NW;
+  // bytes of a lane's two loads within a step: the half line (c & 1), chunk h of it
+  const unsigned lo = 64 * (c & 1) + 16 * h, k2 = 2u * k;
+  const int nr = n - row0 < 16 * RB ? n - row0 : 16 * RB;
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w + (size_t)row0 * k),
+                                                                      (short)0, (int)(nr * k2), kRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), (short)0, (int)(m * k2),
+                                                                      kRsrcWord3);
+  const unsigned v0 = (c & ~1) * k2 + lo;  // the lane's first load: row (token) c & ~1 of a block; the second a row further
+  f32x4 acc[RB][TT];
 #pragma unroll
-  for (int t = 0; t < TT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int steps = (k + 63) >> 6;
-  const uint4 z = make_uint4(0u, 0u, 0u, 0u);
-  // KU of the wave's steps at a time: their weight loads (and with one token tile their activation loads) are issued
-  // together, then their MFMAs in step order -- the same chain as one step at a time
-  constexpr int KU = 4;
-  for (int s0 = wave; s0 < steps; s0 += kWaves * KU) {
-    uint4 a0[KU], a1[KU], b0[KU], b1[KU];
+  for (int r = 0; r < RB; ++r)
 #pragma unroll
-    for (int u = 0; u < KU; ++u) {
-      // unconditional 16-byte loads at clamped (always valid) offsets, zeros selected afterwards: a conditional load
-      // would be split into guarded dword loads
-      const int s = s0 + u * kWaves, k0 = 64 * s;
-      const bool in = s < steps, two = k0 + 32 < k;
-      const int ka = in ? k0 : 0, kb = in && two ? k0 + 32 : 0;
-      const u32x4 va = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wr + ka));
-      const u32x4 vb = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wr + kb));
-      a0[u] = rok && in ? make_uint4(va[0], va[1], va[2], va[3]) : z;
-      a1[u] = rok && in && two ? make_uint4(vb[0], vb[1], vb[2], vb[3]) : z;
-      if constexpr (TT == 1) {
-        const int tok = lane & 15;
-        const uint16_t* xr = x + (size_t)(tok < m ? tok : 0) * k + kq;
-        const uint4 xa = *reinterpret_cast<const uint4*>(xr + ka), xb = *reinterpret_cast<const uint4*>(xr + kb);
-        b0[u] = tok < m && in ? xa : z;
-        b1[u] = tok < m && in && two ? xb : z;
-      }
+    for (int t = 0; t < TT; ++t) acc[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  struct Step {
+    u32x4 a[RB][2], b[TT][2];
+  };
+  // a step's loads; rows past n and tokens past m read zeros (out of the buffers' range), steps past the wave's last
+  // are not used and mostly out of range too
+  auto load = [&](int s, Step& d) __attribute__((always_inline)) {
+    const unsigned v = v0 + (s < s_hi ? 128u * s : 0x40000000u);
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) d.a[r][e] = __builtin_amdgcn_raw_buffer_load_b128(rw, (int)(v + (16 * r + e) * k2), 0, 2);
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) d.b[t][e] = __builtin_amdgcn_raw_buffer_load_b128(rx, (int)(v + (16 * t + e) * k2), 0, 0);
+  };
+  auto use = [&](int s, Step& d) __attribute__((always_inline)) {
+    if (s >= s_hi) return;
+    const bool cut = 64 * s + 32 >= k;
+    const u32x4 z = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      own_row(d.a[r][0], d.a[r][1], odd);
+      if (cut) d.a[r][1] = z;
     }
 #pragma unroll
-    for (int u = 0; u < KU; ++u) {
-      const int s = s0 + u * kWaves, k0 = 64 * s;
-      if (s >= steps) break;
-      const bool two = k0 + 32 < k;  // k % 32 == 0: the step's second slice exists unless k ends at k0 + 32
+    for (int t = 0; t < TT; ++t) {
+      own_row(d.b[t][0], d.b[t][1], odd);
+      if (cut) d.b[t][1] = z;
+    }
 #pragma unroll
-      for (int t = 0; t < TT; ++t) {
-        uint4 xb0 = b0[u], xb1 = b1[u];
-        if constexpr (TT > 1) {
-          const int tok = 16 * t + (lane & 15);
-          const bool tk = tok < m;
-          const uint16_t* xr = x + (size_t)(tk ? tok : 0) * k + kq + k0;
-          const uint4 xa = *reinterpret_cast<const uint4*>(xr), xb = *reinterpret_cast<const uint4*>(xr + (two ? 32 : 0));
-          xb0 = tk ? xa : z;
-          xb1 = tk && two ? xb : z;
-        }
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a0[u]), as_bf16x8(xb0), acc[t], 0, 0, 0);
-        if (two) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a1[u]), as_bf16x8(xb1), acc[t], 0, 0, 0);
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int t = 0; t < TT; ++t)
+#pragma unroll
+        for (int r = 0; r < RB; ++r)
+          acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, d.a[r][e]),
+                                                              __builtin_bit_cast(bf16x8, d.b[t][e]), acc[r][t], 0, 0, 0);
+  };
+  if (s_lo < s_hi) {
+    // two groups of steps in turn, the next one requested before this one is used (no request past the last step: a
+    // branch around the loads alone would make their wait counts conservative, so the last use is a path of its own)
+    Step st[2][KU];
+    auto load_group = [&](int s, Step (&d)[KU]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int u = 0; u < KU; ++u) load(s + u, d[u]);
+    };
+    auto use_group = [&](int s, Step (&d)[KU]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int u = 0; u < KU; ++u) use(s + u, d[u]);
+    };
+    load_group(s_lo, st[0]);
+    if constexpr (TT * RB >= 8) {  // registers for one copy of the uses only: the last requests are past the chunk
+      for (int s = s_lo; s < s_hi; s += 2 * KU) {
+        load_group(s + KU, st[1]);
+        use_group(s, st[0]);
+        load_group(s + 2 * KU, st[0]);
+        use_group(s + KU, st[1]);
       }
+    } else for (int s = s_lo;; s += 2 * KU) {
+      if (s + KU >= s_hi) {
+        use_group(s, st[0]);
+        break;
+      }
+      load_group(s + KU, st[1]);
+      use_group(s, st[0]);
+      if (s + 2 * KU >= s_hi) {
+        use_group(s + KU, st[1]);
+        break;
+      }
+      load_group(s + 2 * KU, st[0]);
+      use_group(s + KU, st[1]);
     }
   }
 #pragma unroll
-  for (int t = 0; t < TT; ++t) red[wave][t][lane] = acc[t];
-  __syncthreads();
-  // thread (tile t, lane) of the first TT waves adds the waves' partials in wave order, then the bias, and writes its
-  // 4 rows of token 16 t + lane % 16
-  if (wave < TT) {
-    const int t = wave;
-    f32x4 v = red[0][t][lane];
+  for (int r = 0; r < RB; ++r)
 #pragma unroll
-    for (int ww = 1; ww < kWaves; ++ww) v += red[ww][t][lane];
-    const int tok = 16 * t + (lane & 15);
+    for (int t = 0; t < TT; ++t) red[(wave * RB * TT + r * TT + t) * 64 + lane] = acc[r][t];
+  __syncthreads();
+  // wave i adds the chunks' partials of tiles i, i + 8, .. in chunk order, then the bias, and writes 4 rows of a token
+  for (int i = wave; i < RB * TT; i += NW) {
+    const int r = i / TT, t = i - r * TT;
+    f32x4 v = red[i * 64 + lane];
+#pragma unroll
+    for (int ww = 1; ww < NW; ++ww) v += red[(ww * RB * TT + i) * 64 + lane];
+    const int tok = 16 * t + c;
     if (tok < m) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int row = (int)blockIdx.x * 16 + 4 * (lane >> 4) + i;
+      for (int e = 0; e < 4; ++e) {
+        const int row = row0 + 16 * r + 4 * h + e;
         if (row < n) {
           const float b = bias ? __uint_as_float((uint32_t)bias[row] << 16) : 0.f;
-          y[(size_t)tok * ldy + row] = f2bf(bias ? v[i] + b : v[i]);
+          y[(size_t)tok * ldy + row] = f2bf(bias ? v[e] + b : v[e]);
         }
       }
     }
   }
+}
+
+template <int TT, int RB, int KU>
+void launch_bi(const uint16_t* x, int m, const uint16_t* w, const uint16_t* bias, uint16_t* y, int n, int k, long ldy,
+               hipStream_t s) {
+  hipLaunchKernelGGL((bi_gemv_kernel<TT, RB, KU>), dim3((n + 16 * RB - 1) / (16 * RB)), dim3(NW * 64),
+                     NW * RB * TT * 64 * sizeof(f32x4), s, x, m, w, bias, y, n, k, ldy);
+}
+
+// Row blocks per workgroup, 1 or 2 (the same results).  Workgroups take rounds of one per CU (two on a CU share its
+// throughput); a round of one-block workgroups takes u, of two-block ones r u, unless the weights' stream is longer,
+// which runs faster with more workgroups (7.3 against 6.0 TB/s).  Measured at k = 5120 (us, one / two blocks): 16 tokens
+// n = 4096 11.5 / 15.7, 5120 19.1 / 15.9, 8192 20.1 / 17.2, 12000 27.7 / 29.2; 1 token n = 20000 33.8 / 36.4; 64 tokens n
+// = 3200 20.8 / 26.6, 4500 36.1 / 26.1; k = 8192, 4 tokens n = 8000 22.0 / 26.9.
+int rows_per_workgroup(int n, int k, int m) {
+  const double u = (m <= 16 ? 5.0 + 2.5 * m / 16 : m <= 32 ? 11.0 : m <= 64 ? 16.5 : 29.0) * k / 5120;
+  const double r = m <= 16 ? 1.5 : m <= 32 ? 1.4 : m <= 64 ? 1.33 : 1.2, bytes = 2.0 * n * k;
+  const int nb = (n + 15) / 16, cus = num_cus();
+  const double one = (nb + cus - 1) / cus * u, two = (nb + 2 * cus - 1) / (2 * cus) * r * u;
+  if (k >= 1 << 24) return 1;  // 32-bit buffer offsets
+  return std::max(two, bytes / 6.0e6) < std::max(one, bytes / 7.3e6) ? 2 : 1;
+}
+
+template <int TT, int KU1, int KU2>
+void launch_rows(const uint16_t* x, int m, const uint16_t* w, const uint16_t* bias, uint16_t* y, int n, int k, long ldy,
+                 hipStream_t s) {
+  if (rows_per_workgroup(n, k, m) == 2)
+    launch_bi<TT, 2, KU2>(x, m, w, bias, y, n, k, ldy, s);
+  else
+    launch_bi<TT, 1, KU1>(x, m, w, bias, y, n, k, ldy, s);
 }
 
 }  // namespace
@@ -130,14 +219,21 @@ extern "C" int ak_bf16_gemv_bi_ld(const void* x, const void* w, const void* bias
   auto W = static_cast<const uint16_t*>(w);
   auto B = static_cast<const uint16_t*>(bias);
   auto Y = static_cast<uint16_t*>(y);
-  const dim3 grid((n + 15) / 16), block(agq::kWaves * 64);
-  const int tt = (m + 15) / 16;
-  switch (tt) {
-    case 1: hipLaunchKernelGGL(agq::bi_gemv_kernel<1>, grid, block, 0, s, X, m, W, B, Y, n, k, ldy); break;
-    case 2: hipLaunchKernelGGL(agq::bi_gemv_kernel<2>, grid, block, 0, s, X, m, W, B, Y, n, k, ldy); break;
-    case 3:
-    case 4: hipLaunchKernelGGL(agq::bi_gemv_kernel<4>, grid, block, 0, s, X, m, W, B, Y, n, k, ldy); break;
-    default: hipLaunchKernelGGL(agq::bi_gemv_kernel<8>, grid, block, 0, s, X, m, W, B, Y, n, k, ldy); break;
+  // 32-bit buffer offsets: as many tokens per launch as they cover (all of them below k = 2^24)
+  if (k >= 1 << 27) return AK_INVALID;
+  const int most = k < 1 << 24 ? 128 : 16;
+  for (int m0 = 0; m0 < m; m0 += most) {
+    const int mm = m - m0 < most ? m - m0 : most;
+    const uint16_t* x0 = X + (size_t)m0 * k;
+    uint16_t* y0 = Y + (size_t)m0 * ldy;
+    const int tt = (mm + 15) / 16;
+    switch (tt) {
+      case 1: agq::launch_rows<1, 2, 2>(x0, mm, W, B, y0, n, k, ldy, s); break;
+      case 2: agq::launch_rows<2, 2, 2>(x0, mm, W, B, y0, n, k, ldy, s); break;
+      case 3:
+      case 4: agq::launch_rows<4, 1, 1>(x0, mm, W, B, y0, n, k, ldy, s); break;
+      default: agq::launch_rows<8, 1, 1>(x0, mm, W, B, y0, n, k, ldy, s); break;
+    }
   }
   return (int)hipGetLastError();
 }

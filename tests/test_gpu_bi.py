@@ -43,6 +43,21 @@ def test_exact_integer_operands(m, n, k, with_bias):
     assert np.array_equal(got, want), f"{int(np.sum(got != want))} of {got.size} differ"
 
 
+# one and two 16-row blocks per workgroup (n up to and over 256 blocks) for each number of token tiles, ragged rows in
+# the last workgroup, chunks of k without a step, with one, and with an odd number of steps, and a last half step
+@pytest.mark.parametrize("m,n,k", [(1, 4097, 32), (16, 4500, 96), (7, 8190, 544), (17, 4100, 1056), (32, 333, 416),
+                                   (33, 4130, 736), (64, 4096, 160), (65, 4200, 608), (128, 5121, 1184)])
+def test_exact_integer_operands_over_row_blocks(m, n, k):
+    """Integers with |sum| < 2^24: every order gives the exact product, so each output is its one rounding to bf16."""
+    rng = np.random.default_rng(m + n + k)
+    xi, wi = rng.integers(-4, 5, size=(m, k)), rng.integers(-8, 9, size=(n, k))
+    b = rng.integers(-64, 65, size=n)
+    got = run(f2bf_array(xi.astype(np.float32).ravel()), f2bf_array(wi.astype(np.float32).ravel()),
+              f2bf_array(b.astype(np.float32)), m, n, k, ldy=n + 5).reshape(m, n + 5)
+    want = f2bf_array((xi.astype(np.float32) @ wi.astype(np.float32).T + b).ravel()).reshape(m, n)
+    assert np.array_equal(got[:, :n], want) and np.all(got[:, n:] == 0x7FC1)
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 24, 5120), (8, 48, 7168), (33, 200, 3072)])
 def test_within_fp32_accumulation_tolerance(m, n, k):
     rng = np.random.default_rng(n + k)
