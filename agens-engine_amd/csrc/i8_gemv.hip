@@ -9,13 +9,16 @@
 // Layout on MI355X: a half-wave (32 lanes) plays the reference's warp for kRows rows at once (the lanes' chunk loads
 // of a row are 512 contiguous bytes, one 16-byte non-temporal load per lane); the activations' chunk is loaded once
 // per token and applied to all of the half-wave's rows (4 for one token, else 2).  A workgroup of 256 threads is 8
-// half-waves.  The weight stream is
+// half-waves.  Two to 16 tokens whose activations fit: i8_gemv_lds_kernel below.  The weight stream is
 // the only large traffic: at m = 1 the kernel is bounded by HBM (1 byte per weight), from about m = 4 on by the
 // VALU (one fma per weight and token).
 #include "agens_kernels.h"
 #include "wq_common.h"
 
 namespace agq {
+
+int num_cus();
+
 namespace {
 
 // rows per half-wave: 4 for one token (the activation chunk's conversion shared by more rows), 2 with more tokens
@@ -134,6 +137,142 @@ __global__ void __launch_bounds__(256) i8_gemv_kernel(const uint16_t* __restrict
   }
 }
 
+constexpr int kRsrcWord3 = 0x00020000;  // raw buffer resource, dword 3 (CDNA)
+
+// The same sums for MT tokens with their activations in LDS: persistent workgroups that take groups of 8 R rows (R per
+// half-wave) in turn.  With the activations read from memory, every token's chunk was waited for in order behind the
+// next weights, which drained the weight stream once per chunk; here the next chunk's weights (of the next group at a
+// group's end) are the only loads outstanding, and they stay in flight over a whole chunk.  A token's chunk is read from
+// LDS while the chains of the token before run (two planes of 16-byte halves: no bank conflicts) and is unpacked once
+// for R rows.  What is left is the VALU: per weight MT fmas (the reference's order), one conversion and MT / R unpacking
+// operations; at 4 tokens and R = 4 about 125 us of the 148 measured for 152064 x 5120, at 8 tokens nearly
+// all of the 228.
+template <int MT, int R>
+__global__ void __launch_bounds__(256, R == 4 ? 3 : 4) i8_gemv_lds_kernel(
+    const uint16_t* __restrict__ x, const int8_t* __restrict__ w, const float* __restrict__ scale,
+    uint16_t* __restrict__ y, int n, int k, int ldy) {
+  constexpr int NV = R * MT, GR = 8 * R;
+  extern __shared__ __attribute__((aligned(16))) u32x4 xs[];  // [token][chunk half][chunk]
+  const int chunks = k >> 4;
+  for (int i = threadIdx.x; i < MT * chunks * 2; i += 256) {
+    const int t = i / (2 * chunks), p = i - t * 2 * chunks;
+    xs[(t * 2 + (p & 1)) * chunks + (p >> 1)] = reinterpret_cast<const u32x4*>(x)[i];
+  }
+  __syncthreads();
+  const int l = threadIdx.x & 31, hw = threadIdx.x >> 5;
+  const int groups = (n + GR - 1) / GR, iters = (chunks + 31) >> 5;
+  auto rows_of_group = [&](int g) __attribute__((always_inline)) {
+    const int g1 = g < groups ? g : (int)blockIdx.x;  // past the end: the first group again, not used
+    const int nr = n - g1 * GR < GR ? n - g1 * GR : GR;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(w + (size_t)g1 * GR * k), (short)0, nr * k, kRsrcWord3);
+  };
+  const int vo = hw * R * k + l * 16;
+  u32x4 nx[R];
+  auto fetch = [&](int g, int it) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t rw = rows_of_group(g);
+#pragma unroll
+    for (int r = 0; r < R; ++r) nx[r] = __builtin_amdgcn_raw_buffer_load_b128(rw, vo + r * k + it * 512, 0, 2);
+  };
+  // the value (row idx % R, token idx / R) that this lane ends with (the reduction below), and whether it writes it
+  constexpr int NP = NV <= 2 ? 2 : NV <= 4 ? 4 : NV <= 8 ? 8 : NV <= 16 ? 16 : 32;  // values padded to a power of two
+  int idx = 0;
+#pragma unroll
+  for (int st = 0; st < 5; ++st) idx += l & (16 >> st) ? NP >> st >> 1 : 0;
+  const bool wr = idx < NV && (l & (32 / NP - 1)) == 0;
+  fetch(blockIdx.x, 0);
+  for (int g = blockIdx.x; g < groups; g += gridDim.x) {
+    const int o = g * GR + hw * R + idx % R;
+    const float sc = scale[o < n ? o : n - 1];
+    float acc[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) acc[i] = 0.f;
+    for (int it = 0; it < iters; ++it) {
+      float qf[R][16];
+#pragma unroll
+      for (int r = 0; r < R; ++r) chunk_f32(make_uint4(nx[r][0], nx[r][1], nx[r][2], nx[r][3]), qf[r]);
+      const bool last = it + 1 == iters;
+      fetch(last ? g + (int)gridDim.x : g, last ? 0 : it + 1);
+      const int c = it * 32 + l;
+      if (c < chunks) {
+        // the next token's chunk is read while this one's chains run
+        u32x4 a = xs[c], b = xs[chunks + c];
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+          const u32x4 ca = a, cb = b;
+          if (j + 1 < MT) a = xs[(2 * j + 2) * chunks + c], b = xs[(2 * j + 3) * chunks + c];
+          float xf[16];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            xf[2 * i] = bf_lo(ca[i]), xf[2 * i + 1] = bf_hi(ca[i]);
+            xf[8 + 2 * i] = bf_lo(cb[i]), xf[9 + 2 * i] = bf_hi(cb[i]);
+          }
+          float s[R];
+#pragma unroll
+          for (int r = 0; r < R; ++r) s[r] = 0.f;
+#pragma unroll
+          for (int e = 0; e < 16; ++e)
+#pragma unroll
+            for (int r = 0; r < R; ++r) s[r] = __builtin_fmaf(xf[e], qf[r][e], s[r]);
+#pragma unroll
+          for (int r = 0; r < R; ++r) acc[j * R + r] += s[r];
+        }
+      }
+    }
+    // the butterfly over the 32 lanes, each step exchanging the half of the values that the partner keeps (both lanes of
+    // a pair would form the same sum): lane l ends with the values of the index bits its lane bits stand for
+#pragma unroll
+    for (int st = 0; st < 5; ++st) {
+      const int d = 16 >> st, cnt = NP >> st >> 1;  // values left after this step
+      if (cnt >= 1) {
+        const bool up = l & d;
+#pragma unroll
+        for (int i = 0; i < cnt; ++i) {
+          const float lo = i < NV ? acc[i] : 0.f, hi = i + cnt < NV ? acc[i + cnt < NV ? i + cnt : 0] : 0.f;
+          acc[i < NV ? i : 0] = (up ? hi : lo) + __shfl_xor(up ? lo : hi, d, 32);
+        }
+      } else {
+        acc[0] += __shfl_xor(acc[0], d, 32);
+      }
+    }
+    if (o < n && wr) y[(size_t)(idx / R) * ldy + o] = f2bf(acc[0] * sc);
+  }
+}
+
+template <int MT, int R>
+void launch_lds(const uint16_t* x, const int8_t* w, const float* scale, uint16_t* y, int n, int k, int ldy,
+                hipStream_t s) {
+  // as many workgroups per CU as the LDS and the registers (3 of 4 rows, 4 of 2 rows per half-wave) take
+  const size_t smem = (size_t)MT * k * 2, fit = (size_t)160 * 1024 / smem;
+  const int per = fit < (R == 4 ? 3 : 4) ? (int)fit : (R == 4 ? 3 : 4);
+  const int groups = (n + 8 * R - 1) / (8 * R), grid = groups < num_cus() * per ? groups : num_cus() * per;
+  hipLaunchKernelGGL((i8_gemv_lds_kernel<MT, R>), dim3(grid), dim3(256), smem, s, x, w, scale, y, n, k, ldy);
+}
+
+template <int MT>
+void launch_lds_rows(const uint16_t* x, const int8_t* w, const float* scale, uint16_t* y, int n, int k, int ldy,
+                     hipStream_t s) {
+  // 2 rows per half-wave where 4 leave CUs idle (8001 x 1040, 8 tokens 8.2 against 9.2 us; 20000 x 2000 18.7 / 19.5;
+  // 152064 x 5120 274 / 233)
+  if (n < 32768)
+    launch_lds<MT, 2>(x, w, scale, y, n, k, ldy, s);
+  else
+    launch_lds<MT, 4>(x, w, scale, y, n, k, ldy, s);
+}
+
+void lds_part(const uint16_t* x, const int8_t* w, const float* scale, uint16_t* y, int m, int n, int k, int ldy,
+              hipStream_t s) {
+  switch (m) {
+    case 1: return launch_lds_rows<1>(x, w, scale, y, n, k, ldy, s);
+    case 2: return launch_lds_rows<2>(x, w, scale, y, n, k, ldy, s);
+    case 3: return launch_lds_rows<3>(x, w, scale, y, n, k, ldy, s);
+    case 4: return launch_lds_rows<4>(x, w, scale, y, n, k, ldy, s);
+    case 5: return launch_lds_rows<5>(x, w, scale, y, n, k, ldy, s);
+    case 6: return launch_lds_rows<6>(x, w, scale, y, n, k, ldy, s);
+    case 7: return launch_lds_rows<7>(x, w, scale, y, n, k, ldy, s);
+    default: return launch_lds_rows<8>(x, w, scale, y, n, k, ldy, s);
+  }
+}
+
 }  // namespace
 }  // namespace agq
 
@@ -147,6 +286,18 @@ extern "C" int ak_i8_gemv(const void* x, const void* w, const void* scale, void*
   auto S = static_cast<const float*>(scale);
   auto Y = static_cast<uint16_t*>(y);
   auto wgs = [n](int rows) { return dim3((n + 8 * rows - 1) / (8 * rows)); };  // 8 half-waves per workgroup
+  // Two to 16 tokens in parts of at most 8 whose activations take at most 80 KB of LDS (two workgroups per CU): the LDS
+  // kernel where at most two parts, i.e. two passes over the weights, cover them.  Measured (us, 152064 x 5120, before =
+  // activations from L1 per token and row pair): 2 / 4 / 8 / 16 tokens 156 / 233 / 358 / 628 -> 119 / 148 / 228 / 460.
+  // Two or three tokens on less than 32 MB of weights stay with the kernel below (8001 x 1040: 7.1 against 7.4, 7.4
+  // against 7.7).
+  const int cap = 81920 / (2 * k), most = cap < 8 ? cap : 8;
+  if (m > 1 && most > 0 && m <= 2 * most && (m > 3 || (long long)n * k >= 32 << 20)) {
+    const int parts = (m + most - 1) / most, per = (m + parts - 1) / parts;
+    for (int m0 = 0; m0 < m; m0 += per)
+      agq::lds_part(X + (size_t)m0 * k, W, S, Y + (size_t)m0 * ldy, m - m0 < per ? m - m0 : per, n, k, ldy, s);
+    return (int)hipGetLastError();
+  }
   if (m == 1 && k <= 16384)
     hipLaunchKernelGGL((agq::i8_gemv_kernel<1, true>), wgs(agq::rows_of<1>()), dim3(256), 0, s, X, W, S, Y, m, n, k,
                        ldy);

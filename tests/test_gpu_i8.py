@@ -43,6 +43,22 @@ def test_matches_oracle_bit_exact(m, n, k):
     assert np.array_equal(got, want), f"{int(np.sum(got != want))} of {got.size} outputs differ"
 
 
+# 2 to 16 tokens with the activations in LDS: 2 and 4 rows per half-wave (n below and from 32768), every number of
+# tokens of a part, one and two parts, rows past the last group, chunks that do not fill the 32 lanes; the last two
+# shapes' activations do not fit (the kernel that reads them from memory)
+@pytest.mark.parametrize("m,n,k", [(2, 32771, 1040), (3, 32768, 1040), (4, 32799, 16), (5, 32801, 1600), (6, 33000, 512),
+                                   (7, 32769, 144), (8, 32770, 2064), (2, 2049, 16400), (4, 515, 5120), (6, 31, 48),
+                                   (7, 300, 1040), (8, 1, 5120), (11, 40, 5120), (13, 32775, 528), (16, 97, 4112),
+                                   (16, 40, 5136), (3, 33, 20496)])
+def test_tokens_in_lds_match_oracle_bit_exact(m, n, k):
+    x, q, scale = data(40 + m + n, m, n, k)
+    ldy = n + 3
+    got = run(x, q, scale, m, n, k, ldy=ldy).reshape(m, ldy)
+    want = ora(x, q, scale, m, n, k, ldy).reshape(m, ldy)
+    assert np.array_equal(got[:, :n], want[:, :n]), f"{int(np.sum(got[:, :n] != want[:, :n]))} outputs differ"
+    assert np.all(got[:, n:] == 0x7FC1), "columns past n were written"
+
+
 def test_order_known_answer_on_gpu():
     """The hand-computed order case of the oracle tests: the reference's order gives 2 (a left-to-right sum 1)."""
     k = 16 * 64
