@@ -23,6 +23,7 @@ int exact_ct_gemv(const void* x, const int32_t* packed, const void* scales, void
 int i8_gemv(int bits, const void* x, int m, const Segs& g, int k, int group, hipStream_t s);
 int i8_gemv_m1(int bits, const void* x, int m, const Segs& g, int k, int group, hipStream_t s, int act = 0);
 int i8_gemv_mt(int bits, const void* x, int m, const Segs& g, int k, int group, hipStream_t s, int act = 0);
+int tile_gemv(int bits, const void* x, int m, const Segs& g, int k, int group, hipStream_t s, int act);
 int mm_gemv(int bits, const void* x, int m, const Segs& g, int k, int group, hipStream_t s, int act);
 int m1d_chain_make(int nsteps, const int* bits, const void* const* x, const int* m, const int* k, const Segs* segs,
                    const int* wait, const int* act, void** table, int* mt_out, size_t* smem_out);
@@ -54,8 +55,8 @@ bool exact_mode() {
   return env == 1;
 }
 
-// The smallest token count routed to the fp16-MFMA kernel (wq_mm.hip) in the default numerics: the measured crossover
-// with the integer-limb kernels (below it those are faster).  Both compute the same numerics bit for bit, so the
+// The smallest token count routed to the fp16-MFMA kernel (wq_mm.hip) in the default numerics, where the tiled kernel
+// (tile_route) does not take the call: the measured crossover with the integer-limb kernels (below it those are faster).  Both compute the same numerics bit for bit, so the
 // switch changes speed only.  0: never; set through ak_wq_set_mm_min or AGENS_WQ_MM_MIN.  Above kMmMaxK inputs the
 // integer kernels stay faster at every token count (measured: down 5120 x 27648 at 24..128 tokens).
 constexpr int kMmMinDefault = 17;
@@ -81,6 +82,28 @@ bool mm_route(int m, int k, int group, bool exact) {
   const int set = mm_min_set();
   if (set >= 0) return set > 0 && m >= set;
   return m >= kMmMinDefault && k <= kMmMaxK;
+}
+
+// Whether a default-numerics call takes the tiled kernel (wq_tile.hip; same bits).  An explicit crossover keeps the older
+// kernels.  Measured, the older kernels' time -> the tiled kernel's, us:
+//   group 64 (which the small-M kernels do not take), every token count: 5120 x 6144 W4 28 -> 18 at 1 token, 188 -> 19 at
+//     16; 55296 x 5120 W3 84 -> 66 and 624 -> 70; 152064 x 5120 W4 153 -> 127 at 1; 22000 x 2560 W3 34.1 -> 33.9 at 1
+//     (the smallest gain met); 64 x 64 14.8 -> 11.1;
+//   group 128 from 33 tokens: 55296 x 5120 W3 164 -> 86 at 64 tokens, 5120 x 5120 W4 38.6 -> 28.9, 5120 x 27648 W3 130 ->
+//     68, 64 x 512 19.8 -> 12.3; at 17 to 32 tokens on wide linears, 55296 x 5120 W3 82 -> 60, 14000 x 2560 W3 29.4 -> 22,
+//     7168 x 5120 W4 25.9 -> 24.2 at 17, but 5120 x 5120 W4 19.7 -> 20.4 and 1000 x 2048 W3 12.5 -> 13.6: the fp16-MFMA
+//     kernel up to kTileRows rows; past kMmMaxK inputs, where the other side is the integer kernels in chunks of 16
+//     tokens, from 24: 5120 x 27648 W2 51.9 -> 47.4 at 24, 45.5 -> 47.3 at 20;
+//   up to 16 tokens at group 128 the small-M kernels (55296 x 5120 W3, 16 tokens: 46 against 49).
+constexpr int kTileRows = 6144;
+bool tile_route(int m, const Segs& g, int k, int group, bool exact) {
+  if (exact || mm_min_set() >= 0) return false;
+  if (group == 64 || m > 32) return true;
+  if (m <= 16) return false;
+  if (k > kMmMaxK) return m >= 24;
+  long long rows = 0;
+  for (int i = 0; i < g.nseg; ++i) rows += g.n[i];
+  return rows > kTileRows;
 }
 
 bool group_ok(int k, int group) { return (group == 64 || group == 128) && k % group == 0 && k % 32 == 0; }
@@ -155,8 +178,13 @@ int gemv(int bits, const void* x, int m, int nseg, const void* const* wt, const 
   const bool exact = bf16w || (!force_default && exact_mode());
   if (act && exact) return AK_INVALID;  // the fused activation is in the default path's kernels only
   std::lock_guard<std::mutex> lock(scratch_mutex(s));
+  const Segs all = make_segs(nseg, wt, st, y, n, ldy, 16);
+  if (tile_route(m, all, k, group, exact)) {
+    const int e = tile_gemv(bits, x, m, all, k, group, s, act);
+    if (e != AK_INVALID) return e;
+  }
   if (mm_route(m, k, group, exact)) {  // above the crossover: the fp16-MFMA kernel, all tokens at once
-    const int e = mm_gemv(bits, x, m, make_segs(nseg, wt, st, y, n, ldy, 16), k, group, s, act);
+    const int e = mm_gemv(bits, x, m, all, k, group, s, act);
     if (e != AK_INVALID) return e;
   }
   for (int m0 = 0; m0 < m; m0 += kMaxTokensPerLaunch) {
@@ -198,7 +226,8 @@ int run_step(const ak_wq_step& st, hipStream_t s) {
 
 // ---- the entry point that allocates nothing: split-K partials and counters in a static device array
 //
-// Bytes of split-K scratch the call's route can ask for: 4 KB of row-range counters, then P (<= 8) stripe partials per
+// Bytes of split-K scratch the call's route can ask for (the tiled kernel's partials and activations are no part of it:
+// where they do not fit the array, the call takes the route below it): 4 KB of row-range counters, then P (<= 8) stripe partials per
 // token per output row (rows padded to 16-row blocks), 4 bytes each.  Tokens per launch: the integer kernels take at
 // most 16 (padded to T = 4, 8 or 16: their token groups), the fp16-MFMA route (default numerics, group 128, m at or
 // above its crossover) 16 or 32 (one or two 16-token tiles); chunks of tokens reuse the scratch in stream order.

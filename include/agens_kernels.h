@@ -12,12 +12,14 @@
  *   - `stream` is a hipStream_t (NULL = the default stream); launches are asynchronous and stream-ordered;
  *   - bf16 tensors are passed as void* (raw 16-bit patterns), the int4 container as int32_t words;
  *   - the caller owns every buffer it passes.  The GEMV entry points (and ak_wq_gemm_kt on narrow linears) own scratch
- *     only for split-K launches (long k, or few rows per CU, at more than two tokens or long k): per (device, stream),
+ *     for split-K launches (long k, or few rows per CU, at more than two tokens or long k) and for the converted
+ *     activations of the tiled kernel (default numerics at group 64 or more than 16 tokens): per (device, stream),
  *     allocated zero-filled on the first such call outside a stream capture (that call synchronizes the device once),
  *     grown (at least doubling) when a larger launch needs it; every buffer, a replaced one included, is held until
  *     the process ends -- as the reference's split-K scratch (w4_gemv.cu:2096-2118) -- so graphs captured before a
- *     growth stay valid.  Inside a capture they never allocate or synchronize: without scratch they take a launch
- *     that needs none (the GEMV: same results; the GEMM: k not split), so they can be captured in a hipGraph.
+ *     growth stay valid (graphs captured from one stream share its scratch: run them in order).  Inside a capture they
+ *     never allocate or synchronize: without scratch they take a launch that needs none (the GEMV: same results; the
+ *     GEMM: k not split), so they can be captured in a hipGraph.
  */
 #pragma once
 #include <stddef.h>
@@ -86,8 +88,9 @@ int ak_wq_gemv_kt_multi(int bits, const void* x, int m, int nseg, const void* co
                         void* stream);            /* agens_kernels.h:258-259, w4_gemv.cu:852-876 */
 /* No counterpart in the reference: ak_wq_gemv_kt_multi that allocates nothing, for callers that cannot call hipMalloc
  * (code under stream capture, tight serving loops, harnesses that forbid allocation).  Same arguments, results and
- * error codes; its split-K launches keep their partials and counters in a static 64 MiB device array of the library
- * (one per GPU, held until the process ends) instead of per-stream scratch.  Returns 1 when the call's worst-case
+ * error codes; its launches keep their partials, counters and converted activations in a static 64 MiB device array of
+ * the library (one per GPU, held until the process ends) instead of per-stream scratch, and take the kernels that need
+ * less where the tiled kernel's do not fit.  Returns 1 when the call's worst-case
  * scratch on its route, 4096 + 64 * P * T * sum_i ceil(n[i] / 16) bytes (P = min(8, ceil(k / 1024)); T = 4, 8 or 16
  * for up to 4, 8 or 16 tokens on the integer kernels, 16 or 32 for up to 16 or more tokens on the fp16-MFMA route that
  * the default numerics take from 17 tokens at k <= 8192), exceeds it (e.g. a 152064-row linear at more than 8 tokens).
