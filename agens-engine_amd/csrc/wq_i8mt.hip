@@ -47,6 +47,7 @@ constexpr int kG = 128;
 constexpr int kRsrcWord3 = 0x00020000;  // raw buffer resource, dword 3 (CDNA)
 constexpr int kNt = 2;                    // streaming (non-temporal) cache policy for the weights
 constexpr int kVmcnt0 = 0x0F70;            // s_waitcnt immediate: vector memory counter 0, the others unconstrained
+constexpr int kNoX = 0x3FFFF000;           // an element offset past every activation buffer
 constexpr int kSc1 = 16;                  // device-scope coherent access (sc1): misses / writes through the L2
 
 // Chained launches of this kernel's steps (3..4 tokens): one persistent workgroup per CU runs the steps in order.  A
@@ -201,30 +202,35 @@ __device__ __forceinline__ void mt_body(const I8Args& a, uint8_t* lds, bool wait
   const int g0 = CH || SK ? 4 * stripe_begin(cpa, nquad, P, 2) : 0;
   const int cg = CH || SK ? 4 * stripe_begin(cpb, nquad, P, 2) - g0 : ngroups;
 
-  // ---- activations, step 1: this lane's bf16 inputs (unit u = (token u / cg, group g0 + u % cg)), requested and
-  // waited for before any weight request
+  // ---- activations, step 1: this lane's bf16 inputs (unit u = (token u / cg, group g0 + u % cg)), requested before any
+  // weight and waited for after the first weights' requests (nothing consumes them up to there: a selection of zeros
+  // for lanes without a unit would wait at once), so that the two round trips to memory overlap.  Measured, us: qkv 5120 +
+  // 2 x 1024 x 5120 W4 at 8 tokens 13.0 -> 12.4, 5120 x 5120 W3 at 3 11.1 -> 10.4, 5120 x 27648 W2 at 8 22.1 -> 21.4,
+  // 152064 x 5120 W4 at 8 75.2 -> 68.2, 14000 x 1152 W3 at 16 14.0 -> 13.1
   const int sub = lane % LPU, units = cg * mm, ustride = nwv * UPW;  // real tokens only (padding rows unused)
   const int u0 = wave * UPW + lane / LPU;
   const int npass = (units + ustride - 1) / ustride;
-  uint4 xv[XB];
+  uint4 xv[XB], xu[ACT ? XB : 1];
   // chained: x (the step's activations, mm x k) read device-coherently, or its tagged copy a.xtg (the same layout in
   // 32-bit words) polled until every word the wave holds carries the launch's tag
   const __amdgpu_buffer_rsrc_t rx =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(xb), (short)0, mm * k * 2, kRsrcWord3);
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(xb), (short)0, (ACT ? 4 : 2) * mm * k, kRsrcWord3);
   const __amdgpu_buffer_rsrc_t rxt =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(a.xtg), (short)0, mm * k * 4, kRsrcWord3);
   const bool tagged = CHAIN && a.xtg != nullptr;
   const uint32_t tag2 = (tag & kMtTagMask) * 0x10001u;
   (void)rx, (void)rxt, (void)tag2;
-  auto ld_coherent = [&](int o) __attribute__((always_inline)) {
+  // the lane's bf16 of the unit at element offset o (chained: device-coherent)
+  constexpr int kXaux = CHAIN ? kSc1 : 0;
+  auto ld_x = [&](int o) __attribute__((always_inline)) {
     if constexpr (BITS == 4) {
-      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rx, (o + unit_pair_offset<4>(sub, 0)) * 2, 0, kSc1);
+      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rx, (o + unit_pair_offset<4>(sub, 0)) * 2, 0, kXaux);
       return make_uint4(v[0], v[1], v[2], v[3]);
     } else {
       uint32_t v[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        v[q] = __builtin_amdgcn_raw_buffer_load_b32(rx, (o + unit_pair_offset<BITS>(sub, q)) * 2, 0, kSc1);
+        v[q] = __builtin_amdgcn_raw_buffer_load_b32(rx, (o + unit_pair_offset<BITS>(sub, q)) * 2, 0, kXaux);
       return make_uint4(v[0], v[1], v[2], v[3]);
     }
   };
@@ -281,21 +287,25 @@ __device__ __forceinline__ void mt_body(const I8Args& a, uint8_t* lds, bool wait
               __builtin_amdgcn_s_sleep(1);
             }
           } else {
-            const uint4 v = ld_coherent((int)xo);
+            const uint4 v = ld_x((int)xo);
             xv[b] = ok ? v : make_uint4(0u, 0u, 0u, 0u);
           }
-        } else {
-          uint4 v = load_unit<BITS>(xb + xo, sub);
-          if constexpr (ACT) v = silu_mul8(v, load_unit<BITS>(xb + xo + k, sub));
+        } else if constexpr (CH) {
+          const uint4 v = load_unit<BITS>(xb + xo, sub);
           xv[b] = ok ? v : make_uint4(0u, 0u, 0u, 0u);
+        } else {  // (no unit: an offset past the buffer, zeros; the image, in LDS, keeps k far below it)
+          xv[b] = ld_x(ok ? (int)xo : kNoX);
+          if constexpr (ACT) xu[b] = ld_x(ok ? (int)xo + k : kNoX);
         }
       }
     }
   };
   if constexpr (!CHAIN) {
     xload(0);
+    if constexpr (CH) {  // (waited for here: the item loop's registers are short)
 #pragma unroll
-    for (int b = 0; b < XB; ++b) asm volatile("" ::"v"(xv[b].x), "v"(xv[b].y), "v"(xv[b].z), "v"(xv[b].w));
+      for (int b = 0; b < XB; ++b) asm volatile("" ::"v"(xv[b].x), "v"(xv[b].y), "v"(xv[b].z), "v"(xv[b].w));
+    }
   }
 
   // ---- this wave's tasks: stripe set j, quads [qa, qb), blocks b0w, b0w + bstep, ... < nb
@@ -378,6 +388,7 @@ __device__ __forceinline__ void mt_body(const I8Args& a, uint8_t* lds, bool wait
       const int t = live ? u / cg : 0, g = live ? u - t * cg : 0, tg = t >> 2, ui = t & 3;  // g: of the chunk
       const int eg0 = 8 * sub, ch = eg0 >> 5;
       int b0, b1, b2;
+      if constexpr (ACT) xv[b] = silu_mul8(xv[b], xu[b]);
       const int e = convert_unit<BITS>(xv[b], ximg + ((g * 2) * NT + tg) * 768 + ch * 192 + ui * 48, NT * 768,
                                        sub & 3, live, b0, b1, b2);
       if (live) {
