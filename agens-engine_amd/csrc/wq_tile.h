@@ -480,20 +480,22 @@ int tile_launch(const TileArgs& a, const TileShape& t, const void* x, int k, int
   if (const int e = (int)hipGetLastError()) return e;
   const dim3 grid(a.wg_end[a.segs.nseg - 1]);
   const size_t smem = tile_lds(t, G, a.ntt);
-  switch (t.rg * 100 + t.rb * 10 + (t.sk ? 1 : 0)) {
 #define AK_TILE(RG, RB)                                                                                         \
   case RG * 100 + RB * 10:                                                                                      \
     hipLaunchKernelGGL((tile_kernel<BITS, G, RG, RB, false>), grid, dim3(512), smem, s, a);                     \
-    break;                                                                                                      \
+    return (int)hipGetLastError();                                                                              \
   case RG * 100 + RB * 10 + 1:                                                                                  \
     hipLaunchKernelGGL((tile_kernel<BITS, G, RG, RB, true>), grid, dim3(512), smem, s, a);                      \
-    break;
-    AK_TILE(8, 1) AK_TILE(8, 2) AK_TILE(4, 1) AK_TILE(4, 2) AK_TILE(2, 2) AK_TILE(2, 4) AK_TILE(2, 5) AK_TILE(2, 7)
-    AK_TILE(1, 2) AK_TILE(1, 4) AK_TILE(1, 5) AK_TILE(1, 7)
-#undef AK_TILE
+    return (int)hipGetLastError();
+  if constexpr (G == 64) {  // (up to 16 tokens at group 128: other kernels)
+    switch (t.rg * 100 + t.rb * 10 + (t.sk ? 1 : 0)) { AK_TILE(8, 1) AK_TILE(8, 2) }
+  }
+  switch (t.rg * 100 + t.rb * 10 + (t.sk ? 1 : 0)) {
+    AK_TILE(4, 1) AK_TILE(4, 2) AK_TILE(2, 2) AK_TILE(2, 4) AK_TILE(2, 5) AK_TILE(2, 7) AK_TILE(1, 2) AK_TILE(1, 4)
+    AK_TILE(1, 5) AK_TILE(1, 7)
     default: return AK_INVALID;
   }
-  return (int)hipGetLastError();
+#undef AK_TILE
 }
 
 }  // namespace

@@ -49,11 +49,11 @@ TileShape pick_shape(const TileArgs& a, int group) {
 
 }  // namespace
 
-// 1..128 tokens, group 64 or 128; act = 1 (group 128): x is the merged gate_up [m][2k] and the activations SiLU(gate) *
+// 1..128 tokens at group 64, 17..128 at group 128; act = 1 (group 128): x is the merged gate_up [m][2k] and the activations SiLU(gate) *
 // up.  AK_INVALID where the shape does not suit the kernel or the stream has no scratch (the caller falls back).  Works
 // in the stream's scratch: counters, split-K partials, the activation image; two launches, under scratch_mutex(s).
 int tile_gemv(int bits, const void* x, int m, const Segs& g, int k, int group, hipStream_t s, int act) {
-  if (act && group != 128) return AK_INVALID;
+  if (group == 128 ? m <= 16 : act) return AK_INVALID;
   TileArgs a;
   a.segs = g;
   a.m = m;
