@@ -116,19 +116,18 @@ void set_prefill_tile_bytes(size_t bytes) { g_tile_bytes = bytes; }
 namespace {
 int g_prefill_route = -1;  // -1: by shape, 0: dequantized tiles x library GEMM, 1: the fused GEMM
 
-// The fused prefill GEMM (ak_wq_gemm_kt) against dequantized tiles x rocBLAS, measured on MI355X (us per call,
-// bench.py --config prefill and --config xover):
-//   gate_up W3 55296 x 5120:   m = 512: 441 vs 448, m = 2048: 1436 vs 987;
-//   LM head W4 152064 x 5120:  m = 512: 934 vs 1092, m = 2048: 3076 vs 2648;
-//   down W2 5120 x 27648:      m = 512: 239 vs 354, m = 2048: 677 vs 516;
-//   o W4 5120 x 5120:          m = 256:  41 vs  59, m = 512:  58 vs  51;
-//   qkv W4 7168 x 5120:        m = 256:  49 vs  85, m = 512:  70 vs  72.
-// The fused kernel wins on long k and on wide linears up to several hundred tokens and on every linear up to 256
-// tokens (narrow ones split k across workgroups); the library GEMM on narrow short-k linears beyond that and at large
-// m (the fused kernel expands every weight once per token tile).
+// The fused prefill GEMM (ak_wq_gemm_kt) against dequantized tiles x rocBLAS, measured on MI355X (us per call, weights
+// rotated beyond the cache; fused vs library at each m):
+//   gate_up W3 55296 x 5120:  512: 335 vs 397,  768: 467 vs 502,   1024: 624 vs 611,   1536: 921 vs 843;
+//   LM head W4 152064 x 5120: 512: 769 vs 1065, 768: 1096 vs 1229, 1024: 1490 vs 1688, 1280: 1867 vs 1791;
+//   down W2 5120 x 27648:     512: 148 vs 354,  768: 210 vs 479,   1536: 399 vs 531,   2048: 582 vs 530;
+//   o W4 5120 x 5120:         512:  48 vs  49,  768:  60 vs  67,   1024:  73 vs  67;
+//   qkv W4 7168 x 5120:       512:  60 vs  73,  768:  77 vs 103,   1024:  94 vs 113,   1280: 114 vs 97.
+// The fused kernel wins on every linear up to 768 tokens, on the widest up to 1024 and on long k up to 1536; the
+// library GEMM beyond (the fused kernel expands every weight once per token tile).
 bool prefill_fused(int n, int k, int m) {
   if (g_prefill_route >= 0) return g_prefill_route == 1;
-  return m <= 256 || (k >= 16384 && m <= 1024) || (n >= 16384 && m <= (n >= 100000 ? 1024 : 512));
+  return m <= 768 || (k >= 16384 && m <= 1536) || (n >= 100000 && m <= 1024);
 }
 }  // namespace
 
