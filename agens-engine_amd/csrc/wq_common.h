@@ -12,7 +12,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <mutex>
+#include "wq_scratch.h"
 
 namespace agq {
 
@@ -32,19 +32,6 @@ struct Segs {
 };
 
 __host__ __device__ inline int kpad(int k) { return (k + 1023) & ~1023; }
-
-// A fixed scratch buffer that replaces the per-stream library scratch for the calling host thread while `on` (the
-// entry point that allocates nothing installs it around its launches).
-struct ScratchOverride {
-  void* p = nullptr;
-  size_t bytes = 0;
-  bool on = false;
-};
-ScratchOverride& scratch_override();
-
-// Held while a call on stream s enqueues kernels that work in the stream's scratch: calls of two host threads on one
-// stream are then ordered as wholes, also those whose kernels hand data to each other through the scratch.
-std::mutex& scratch_mutex(hipStream_t s);
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));

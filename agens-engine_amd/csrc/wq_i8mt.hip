@@ -39,7 +39,6 @@
 namespace agq {
 
 int num_cus();
-void* stream_scratch(hipStream_t s, size_t bytes);
 
 namespace {
 

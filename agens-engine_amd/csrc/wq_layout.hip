@@ -3,10 +3,6 @@
 // The KT byte layout is the reference's (kernels/src/w4_gemv.cu:13-31, :439-458, :758-790) so weights repacked here
 // are interchangeable with the reference's; the kernels are written for wave64: one thread per 16-byte lane chunk of
 // the output, consecutive threads writing consecutive chunks of a record (fully coalesced stores), grid-stride loops.
-#include <map>
-#include <vector>
-#include <mutex>
-#include <utility>
 
 #include "agens_kernels.h"
 #include "wq_common.h"
@@ -22,56 +18,6 @@ int num_cus() {
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) cus = 256;
   }
   return cus;
-}
-
-// Library scratch per (device, stream), as the reference keeps its split-K partials and counters
-// (w4_gemv.cu:2096-2118): allocated zero-filled on first use and grown (at least doubling) when a launch needs more,
-// never inside a stream capture (null then: the caller takes a path without scratch).  Every buffer handed out is held
-// until the process ends, the replaced ones included, so launches still in flight and graphs captured before a growth
-// keep valid memory.  Launches on one stream are ordered, so they share it safely.  Users keep their counters (the
-// first 4 KB) at zero between launches.
-//
-// A caller that must not allocate (ak_wq_gemv_kt_multi_noalloc) installs a fixed buffer for the calling thread first:
-// then this returns that buffer when it is large enough and null otherwise, and never allocates.
-ScratchOverride& scratch_override() {
-  static thread_local ScratchOverride o;
-  return o;
-}
-
-std::mutex& scratch_mutex(hipStream_t s) {
-  static std::mutex m[64];  // streams share one only by chance of their address
-  return m[(reinterpret_cast<uintptr_t>(s) >> 6) & 63];
-}
-
-void* stream_scratch(hipStream_t s, size_t bytes) {
-  const ScratchOverride& o = scratch_override();
-  if (o.on) return bytes <= o.bytes ? o.p : nullptr;
-  static std::mutex mu;
-  static std::map<std::pair<int, hipStream_t>, std::pair<void*, size_t>> bufs;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-  std::lock_guard<std::mutex> lock(mu);
-  auto& b = bufs[{dev, s}];
-  if (b.first && b.second >= bytes) return b.first;
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
-    (void)hipGetLastError();
-    return nullptr;
-  }
-  // at least double: a replaced buffer is kept, not freed (a graph captured before the growth still addresses it), so
-  // the retired buffers stay below the current one in total
-  size_t want = bytes > ((size_t)4 << 20) ? bytes : ((size_t)4 << 20);
-  if (b.first && want < 2 * b.second) want = 2 * b.second;
-  void* p = nullptr;
-  if (hipMalloc(&p, want) != hipSuccess || hipMemset(p, 0, want) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
-    if (p) (void)hipFree(p);
-    (void)hipGetLastError();
-    return nullptr;
-  }
-  static std::vector<void*> retired;
-  if (b.first) retired.push_back(b.first);
-  b = {p, want};
-  return p;
 }
 
 namespace {

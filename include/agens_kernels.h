@@ -13,7 +13,8 @@
  *   - bf16 tensors are passed as void* (raw 16-bit patterns), the int4 container as int32_t words;
  *   - the caller owns every buffer it passes.  The GEMV entry points (and ak_wq_gemm_kt on narrow linears) own scratch
  *     for split-K launches (long k, or few rows per CU, at more than two tokens or long k) and for the converted
- *     activations of the tiled kernel (default numerics at group 64 or more than 16 tokens): per (device, stream),
+ *     activations of the tiled kernel (default numerics at group 64 or more than 16 tokens): per (device, stream;
+ *     hipStreamPerThread: and host thread),
  *     allocated zero-filled on the first such call outside a stream capture (that call synchronizes the device once),
  *     grown (at least doubling) when a larger launch needs it; every buffer, a replaced one included, is held until
  *     the process ends -- as the reference's split-K scratch (w4_gemv.cu:2096-2118) -- so graphs captured before a
