@@ -1,7 +1,7 @@
 // GEMV entry points of the C ABI: argument rules, routing between the two numerics and token chunking.  Split-K
-// launches keep stripe partials and row-range counters in library scratch (per (device, stream), allocated on first
-// use outside a stream capture; under a capture without it a route without scratch is taken), or, for
-// ak_wq_gemv_kt_multi_noalloc, in a static device array; every other launch is self-contained (partials meet in LDS).
+// launches keep stripe partials and row-range counters in library scratch, the tiled kernel its converted activations as
+// well (wq_scratch.h: without scratch, e.g. in a capture before any other call, a route that needs none is taken), or,
+// for ak_wq_gemv_kt_multi_noalloc, in a static device array; every other launch is self-contained (partials meet in LDS).
 //
 // Argument rules and return codes follow the reference (kernels/src/w4_gemv.cu:702-731, :852-876, :898-935,
 // :3265-3282): group in {64, 128} with k % group == 0, 1 <= nseg <= 4, 1 <= m <= 128; error 1 otherwise.

@@ -425,18 +425,15 @@ int launch_gemm(const void* x, int m, const void* wt, const void* st, void* y, i
   // 32-bit buffer offsets: the weights, scales and inputs must each stay below 2 GB
   if ((long long)kpad(k) / 1024 * n * 128 * BITS >= (1ll << 31) || (long long)m * k * 2 >= (1ll << 31))
     return AK_INVALID;
-  // fp32 partial tiles of a split launch: in the stream's scratch after its first 4 KB (the GEMV kernels' row-range
-  // counters, which stay zero between launches); one pass where the scratch is not available (e.g. first use under
-  // stream capture)
+  // fp32 partial tiles of a split launch: in call_scratch; one pass without it (e.g. a capture before any other call)
   Tiling tl = pick_tiling(m, n, k / kSlab, true);
   float* part = nullptr;
   std::unique_lock<std::mutex> lock;
   if (tl.split > 1) {
     lock = std::unique_lock<std::mutex>(scratch_mutex(s));  // the two kernels of a split launch stay together
-    if (void* z = stream_scratch(s, 4096 + (size_t)tl.split * ((n + 255) / 256) * ((m + tl.T - 1) / tl.T) * 1024 * tl.T))
-      part = reinterpret_cast<float*>(static_cast<uint8_t*>(z) + 4096);
-    else
-      tl = pick_tiling(m, n, k / kSlab, false);
+    part = reinterpret_cast<float*>(
+        call_scratch(s, (size_t)tl.split * ((n + 255) / 256) * ((m + tl.T - 1) / tl.T) * 1024 * tl.T).data);
+    if (!part) tl = pick_tiling(m, n, k / kSlab, false);
   }
   switch (tl.T) {
     case 64: return launch_t<BITS, G, 64>(x, m, wt, st, y, n, ldy, k, s, tl.split, part);

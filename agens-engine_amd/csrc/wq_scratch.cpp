@@ -10,11 +10,18 @@
 // program whose threads come and go holds as many as were alive at once; a buffer that a captured graph addresses is
 // not passed on.
 //
+// Captured calls.  A graph runs whenever and wherever it is launched: beside other graphs captured from the same stream,
+// and beside later calls on it.  The calls of one capture on one stream therefore share a piece of a reserve (call_scratch)
+// that nothing else uses.  The reserve is 256 MB per device, allocated with the first call outside a capture that needs
+// scratch, on whatever stream; a piece is what the largest of its calls needs (a 16-token decode step of 27648 inputs 3
+// MB, 64 tokens 16 MB).  Pieces are not given back: an executable graph updated from another one (hipGraphExecUpdate) goes
+// on addressing the other's pieces after that one is destroyed, and the runtime does not tell.  When the reserve is used
+// up, calls are captured in the form without scratch.  (The split-K launches of the small-M kernels work in stream_scratch
+// under a capture as well, as the reference's do: graphs with such launches captured from one stream run in order.)
+//
 // A caller that must not allocate (ak_wq_gemv_kt_multi_noalloc) installs a fixed buffer for the calling thread first:
-// then stream_scratch returns that buffer when it is large enough and null otherwise, and never allocates.
+// then both functions return that buffer when it is large enough and null otherwise, and never allocate.
 #include "wq_scratch.h"
-
-#include <stdint.h>
 
 #include <atomic>
 #include <map>
@@ -31,10 +38,20 @@ struct Buf {
   bool captured = false;  // handed out under a stream capture
 };
 
+constexpr size_t kCounters = 4096, kReserve = (size_t)256 << 20;
+struct Reserve {
+  uint8_t* p = nullptr;
+  size_t used = 0;
+  bool tried = false;
+};
+
 struct Pool {
   std::mutex mu;
   std::map<std::tuple<int, hipStream_t, uint64_t>, Buf> bufs;  // (device, stream, thread_of(stream))
   std::vector<std::pair<int, Buf>> idle;                       // (device, buffer) of threads that ended
+  std::map<int, Reserve> reserve;                              // by device
+  // (device, stream, thread_of(stream), capture) -> the piece its calls share
+  std::map<std::tuple<int, hipStream_t, uint64_t, unsigned long long>, Buf> pieces;
 };
 
 Pool& pool() {
@@ -128,6 +145,56 @@ void* stream_scratch(hipStream_t s, size_t bytes) {
     return nullptr;
   }
   return replace_with({p, want, false});
+}
+
+CallScratch call_scratch(hipStream_t s, size_t bytes) {
+  CallScratch c;
+  auto in = [&](void* p) {
+    if (p) c.cnt = static_cast<int*>(p), c.data = static_cast<uint8_t*>(p) + kCounters;
+    return c;
+  };
+  bytes += kCounters;
+  if (scratch_override().on) return in(stream_scratch(s, bytes));
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  // (the legacy stream is never captured, and may not be asked while another one is)
+  if (s && s != hipStreamLegacy && hipStreamGetCaptureInfo_v2(s, &cs, &id, nullptr, nullptr, nullptr) != hipSuccess) {
+    (void)hipGetLastError();
+    return c;
+  }
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return c;
+  Pool& P = pool();
+  if (cs == hipStreamCaptureStatusNone) {
+    void* const z = stream_scratch(s, bytes);
+    std::lock_guard<std::mutex> lock(P.mu);
+    Reserve& r = P.reserve[dev];
+    if (z && !r.tried) {
+      r.tried = true;
+      void* p = nullptr;
+      if (hipMalloc(&p, kReserve) == hipSuccess && hipMemset(p, 0, kReserve) == hipSuccess &&
+          hipDeviceSynchronize() == hipSuccess) {
+        r.p = static_cast<uint8_t*>(p);
+      } else {
+        if (p) (void)hipFree(p);
+        (void)hipGetLastError();
+      }
+    }
+    return in(z);
+  }
+  if (cs != hipStreamCaptureStatusActive) return c;
+  const uint64_t thread = thread_of(s);
+  std::lock_guard<std::mutex> lock(P.mu);
+  const std::tuple<int, hipStream_t, uint64_t, unsigned long long> key{dev, s, thread, id};
+  const auto it = P.pieces.find(key);
+  if (it != P.pieces.end() && it->second.bytes >= bytes) return in(it->second.p);
+  Reserve& r = P.reserve[dev];
+  bytes = (bytes + 4095) & ~(size_t)4095;
+  if (!r.p || kReserve - r.used < bytes) return c;
+  void* const p = r.p + r.used;
+  r.used += bytes;
+  P.pieces[key] = {p, bytes, true};  // (a smaller piece of the capture stays with its earlier calls)
+  return in(p);
 }
 
 }  // namespace agq

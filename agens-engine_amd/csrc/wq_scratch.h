@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime_api.h>
 #include <stddef.h>
+#include <stdint.h>
 
 #include <mutex>
 
@@ -22,5 +23,13 @@ std::mutex& scratch_mutex(hipStream_t s);
 
 // The scratch of stream s on the current device, at least `bytes` long; null without it (see wq_scratch.cpp).
 void* stream_scratch(hipStream_t s, size_t bytes);
+
+// The same for a call that may be captured: 4 KB of counters (zero between launches) and `bytes` of data that no other
+// stream and no other graph works in; null pointers without it.
+struct CallScratch {
+  int* cnt = nullptr;
+  uint8_t* data = nullptr;
+};
+CallScratch call_scratch(hipStream_t s, size_t bytes);
 
 }  // namespace agq

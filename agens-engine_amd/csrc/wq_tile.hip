@@ -50,8 +50,8 @@ TileShape pick_shape(const TileArgs& a, int group) {
 }  // namespace
 
 // 1..128 tokens at group 64, 17..128 at group 128; act = 1 (group 128): x is the merged gate_up [m][2k] and the activations SiLU(gate) *
-// up.  AK_INVALID where the shape does not suit the kernel or the stream has no scratch (the caller falls back).  Works
-// in the stream's scratch: counters, split-K partials, the activation image; two launches, under scratch_mutex(s).
+// up.  AK_INVALID where the shape does not suit the kernel or there is no scratch for the call (the caller falls back).  Works
+// in call_scratch: counters, split-K partials, the activation image; two launches, under scratch_mutex(s).
 int tile_gemv(int bits, const void* x, int m, const Segs& g, int k, int group, hipStream_t s, int act) {
   if (group == 128 ? m <= 16 : act) return AK_INVALID;
   TileArgs a;
@@ -71,16 +71,16 @@ int tile_gemv(int bits, const void* x, int m, const Segs& g, int k, int group, h
     for (int i = 0; i < g.nseg; ++i) part += (size_t)a.P * a.ntt * ((g.n[i] + 15) / 16) * 1024;
   constexpr size_t kMaxScratch = (size_t)256 << 20;  // (128 tokens x 27648 inputs x 5120 rows: 33 MB)
   if (4096 + part + a.img_bytes > kMaxScratch) return AK_INVALID;
-  uint8_t* z = static_cast<uint8_t*>(stream_scratch(s, 4096 + part + a.img_bytes));
-  if (!z) return AK_INVALID;
-  a.cnt = reinterpret_cast<int*>(z);
-  a.part = reinterpret_cast<float*>(z + 4096);
-  a.img = z + 4096 + part;
+  const CallScratch z = call_scratch(s, part + a.img_bytes);
+  if (!z.data) return AK_INVALID;
+  a.cnt = z.cnt;
+  a.part = reinterpret_cast<float*>(z.data);
+  uint8_t* const img = z.data + part;
+  a.img = img;
   for (int i = 0, e = 0; i < kMaxSegs; ++i) {
     if (i < g.nseg) e += ((g.n[i] + 15) / 16 + t.rg * t.rb - 1) / (t.rg * t.rb) * (t.sk ? a.P : 1);
     a.wg_end[i] = e;
   }
-  uint8_t* const img = z + 4096 + part;
   return bits == 4   ? tile_launch_w4(a, t, x, k, group, act, img, s)
          : bits == 3 ? tile_launch_w3(a, t, x, k, group, act, img, s)
                      : tile_launch_w2(a, t, x, k, group, act, img, s);

@@ -14,13 +14,17 @@
  *   - the caller owns every buffer it passes.  The GEMV entry points (and ak_wq_gemm_kt on narrow linears) own scratch
  *     for split-K launches (long k, or few rows per CU, at more than two tokens or long k) and for the converted
  *     activations of the tiled kernel (default numerics at group 64 or more than 16 tokens): per (device, stream;
- *     hipStreamPerThread: and host thread),
- *     allocated zero-filled on the first such call outside a stream capture (that call synchronizes the device once),
- *     grown (at least doubling) when a larger launch needs it; every buffer, a replaced one included, is held until
- *     the process ends -- as the reference's split-K scratch (w4_gemv.cu:2096-2118) -- so graphs captured before a
- *     growth stay valid (graphs captured from one stream share its scratch: run them in order).  Inside a capture they
- *     never allocate or synchronize: without scratch they take a launch that needs none (the GEMV: same results; the
- *     GEMM: k not split), so they can be captured in a hipGraph.
+ *     hipStreamPerThread: and host thread), allocated zero-filled on the first such call outside a stream capture (that
+ *     call synchronizes the device once), grown (at least doubling) when a larger launch needs it; every buffer, a
+ *     replaced one included, is held until the process ends -- as the reference's split-K scratch
+ *     (w4_gemv.cu:2096-2118) -- so graphs captured before a growth stay valid.
+ *   - Inside a capture they never allocate or synchronize, so they can be captured in a hipGraph.  The tiled kernel and
+ *     the GEMM work in a piece of a 256 MB reserve per device (allocated with the first call outside a capture that
+ *     needs scratch, on any stream) that belongs to the captured graph: it may run beside other graphs and beside calls
+ *     on the stream it was captured from (not beside itself).  Without a reserve, or with too little of it left, they
+ *     take a launch that needs no scratch (the GEMV: same results; the GEMM: k not split).  The split-K launches of the
+ *     one- to 16-token kernels at group 128 work in the captured stream's own scratch (if it has any): run graphs that
+ *     hold such launches in order with each other and with calls on that stream.
  */
 #pragma once
 #include <stddef.h>

@@ -7,7 +7,6 @@
 #include <functional>
 #include <map>
 #include <mutex>
-#include <set>
 #include <thread>
 #include <vector>
 
@@ -19,7 +18,8 @@ std::mutex fake_mu;
 size_t live_bytes = 0, peak_bytes = 0;
 int mallocs = 0, syncs = 0, failed = 0;
 std::map<void*, size_t> sizes;
-std::set<hipStream_t> capturing;
+std::map<hipStream_t, unsigned long long> capturing;  // stream -> capture
+unsigned long long captures = 0;
 
 bool any_capture() { return !capturing.empty(); }
 void expect(bool ok, const char* what) {
@@ -41,7 +41,7 @@ hipError_t hipDeviceSynchronize(void) {
 hipError_t hipMalloc(void** p, size_t n) {
   std::lock_guard<std::mutex> l(fake_mu);
   expect(!any_capture(), "an allocation while a stream captures");
-  *p = malloc(n);  // (untouched pages cost nothing)
+  *p = calloc(1, n);  // (untouched pages cost nothing)
   sizes[*p] = n, live_bytes += n, ++mallocs;
   if (live_bytes > peak_bytes) peak_bytes = live_bytes;
   return *p ? hipSuccess : hipErrorOutOfMemory;
@@ -59,6 +59,14 @@ hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* st) {
   *st = capturing.count(s) ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
   return hipSuccess;
 }
+hipError_t hipStreamGetCaptureInfo_v2(hipStream_t s, hipStreamCaptureStatus* st, unsigned long long* id, hipGraph_t*,
+                                      const hipGraphNode_t**, size_t*) {
+  std::lock_guard<std::mutex> l(fake_mu);
+  const auto it = capturing.find(s);
+  *st = it != capturing.end() ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+  if (it != capturing.end()) *id = it->second;
+  return hipSuccess;
+}
 }
 
 using namespace agq;
@@ -66,6 +74,8 @@ using namespace agq;
 namespace {
 constexpr size_t MB = (size_t)1 << 20;
 hipStream_t stream(int i) { return reinterpret_cast<hipStream_t>((uintptr_t)0x1000 * (i + 1)); }
+void begin(hipStream_t s) { capturing[s] = ++captures; }
+void end(hipStream_t s) { capturing.erase(s); }
 void in_thread(const std::function<void()>& f) { std::thread(f).join(); }
 
 void one_stream_one_buffer() {
@@ -108,10 +118,10 @@ void per_thread_stream() {
   void* kept = nullptr;
   in_thread([&] {
     kept = stream_scratch(hipStreamPerThread, 1 * MB);
-    capturing.insert(hipStreamPerThread);
+    begin(hipStreamPerThread);
     expect(stream_scratch(hipStreamPerThread, 1 * MB) == kept, "a warmed stream's buffer under capture");
     expect(stream_scratch(hipStreamPerThread, 64 * MB) == nullptr, "no growth under capture");
-    capturing.erase(hipStreamPerThread);
+    end(hipStreamPerThread);
   });
   for (int i = 0; i < 3; ++i)
     in_thread([&] {
@@ -120,11 +130,71 @@ void per_thread_stream() {
     });
   expect(stream_scratch(hipStreamPerThread, 1 * MB) == mine, "and this thread's is still its own");
 }
+
+// [counters, end of data) of every piece handed out so far: no two may meet
+std::vector<std::pair<uint8_t*, uint8_t*>> taken;
+bool apart(const CallScratch& c, size_t bytes) {
+  uint8_t *const lo = reinterpret_cast<uint8_t*>(c.cnt), *const hi = c.data + bytes;
+  bool ok = c.data >= lo + 4096;
+  for (auto& t : taken) ok = ok && (hi <= t.first || t.second <= lo);
+  taken.push_back({lo, hi});
+  return ok;
+}
+
+void captured_calls() {
+  begin(stream(7));
+  expect(!call_scratch(stream(7), 1 * MB).data, "a capture before any other call has no scratch");
+  end(stream(7));
+  const CallScratch eager = call_scratch(stream(8), 1 * MB);
+  expect(eager.data && eager.data == reinterpret_cast<uint8_t*>(eager.cnt) + 4096, "a call's scratch: counters, data");
+  expect(static_cast<void*>(eager.cnt) == stream_scratch(stream(8), 1 * MB), "outside a capture: the stream's");
+  expect(apart(eager, 1 * MB), "first");
+  const size_t before = live_bytes;
+  // from the warmed stream and from one that the library has not seen, one after the other and at once
+  for (int round = 0; round < 2; ++round) {
+    begin(stream(8));
+    begin(stream(9));
+    const CallScratch a = call_scratch(stream(8), 1 * MB), b = call_scratch(stream(9), 2 * MB);
+    expect(a.data && b.data && apart(a, 1 * MB) && apart(b, 2 * MB), "a captured call shares with nothing else");
+    expect(call_scratch(stream(8), 1 * MB).data == a.data && call_scratch(stream(9), 1 * MB).data == b.data,
+           "the calls of one capture on one stream share");
+    const CallScratch more = call_scratch(stream(8), 5 * MB);
+    expect(more.data && apart(more, 5 * MB), "a larger call of a capture gets a larger piece");
+    expect(call_scratch(stream(8), 1 * MB).data == more.data, "which the later ones share");
+    end(stream(8));
+    end(stream(9));
+    expect(call_scratch(stream(8), 1 * MB).data == eager.data, "calls outside a capture keep the stream's");
+  }
+  begin(stream(8));
+  begin(hipStreamPerThread);
+  CallScratch here = call_scratch(hipStreamPerThread, 1 * MB), there;
+  in_thread([&] { there = call_scratch(hipStreamPerThread, 1 * MB); });
+  expect(apart(here, 1 * MB) && apart(there, 1 * MB), "hipStreamPerThread: by thread");
+  end(hipStreamPerThread);
+  // the fixed buffer of the entry point that allocates nothing comes first
+  static uint8_t fixed[64 << 10];
+  scratch_override() = {fixed, sizeof(fixed), true};
+  expect(static_cast<void*>(call_scratch(stream(8), 60 << 10).cnt) == fixed, "the fixed buffer");
+  expect(!call_scratch(stream(8), 64 << 10).data, "which is too small for 64 KB beside the counters");
+  scratch_override() = ScratchOverride();
+  end(stream(8));
+  // the reserve ends; then there is none, and nothing new was allocated
+  int got = 0;
+  for (int i = 0; i < 400; ++i) {
+    begin(stream(11));
+    const CallScratch c = call_scratch(stream(11), 1 * MB);
+    if (c.data) expect(apart(c, 1 * MB), "pieces are apart to the end"), ++got;
+    end(stream(11));
+  }
+  expect(got > 200 && got < 256, "256 MB in all");
+  expect(live_bytes <= before + 4 * MB + 8 * MB, "captured calls allocate nothing");
+}
 }  // namespace
 
 int main() {
   one_stream_one_buffer();
   per_thread_stream();
+  captured_calls();
   if (!failed) printf("scratch: all checks passed\n");
   return failed ? 1 : 0;
 }

@@ -80,3 +80,52 @@ def test_two_threads_on_the_per_thread_stream(gpu, group, bits, m, n, k):
     assert not any(rcs)
     for c in calls:
         assert np.array_equal(c.out(), c.want)
+
+
+def capture(hip, stream, enqueue):
+    graph, exe = vp(), vp()
+    assert hip.hipStreamBeginCapture(stream, ctypes.c_int(1)) == 0
+    rc = enqueue(stream)
+    assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+    check(rc, "under capture")
+    assert hip.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, ctypes.c_size_t(0)) == 0
+    return graph, exe
+
+
+def nodes(hip, graph):
+    n = ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0
+    return n.value
+
+
+@pytest.mark.parametrize("warm", [True, False])
+@pytest.mark.parametrize("group,bits,m,n,k,gemm", [s + (False,) for s in SHAPES] + [(128, 2, 200, 640, 9344, True)])
+def test_two_graphs_and_a_call_at_once(gpu, group, bits, m, n, k, gemm, warm):
+    """Two graphs captured from one stream (that the library has worked on before, or not), replayed on two others while
+    the stream itself runs a third call: several replays, each as the call alone."""
+    K, hip = gpu
+    calls = [Call(K, 300 + 10 * i, group, bits, m, n, k, gemm) for i in range(3)]
+    streams = [vp() for _ in range(3)]
+    for s in streams:
+        assert hip.hipStreamCreate(ctypes.byref(s)) == 0
+    if warm:
+        check(calls[2].enqueue(streams[2]))
+        assert hip.hipStreamSynchronize(streams[2]) == 0
+    graphs = [capture(hip, streams[2], c.enqueue) for c in calls[:2]]
+    assert all(nodes(hip, g) == 2 for g, _ in graphs), "the two kernels of the route that needs scratch"
+    check(calls[2].enqueue(streams[2]))  # (its first call allocates and synchronizes)
+    for rep in range(4):
+        for c in calls:
+            c.clear()
+        check(K.ak_synchronize())
+        for _ in range(8):
+            for (_, e), s in zip(graphs, streams):
+                assert hip.hipGraphLaunch(e, s) == 0
+            check(calls[2].enqueue(streams[2]))
+        for i, c in enumerate(calls):
+            assert np.array_equal(c.out(), c.want), f"replay {rep}, call {i}"
+    for g, e in graphs:
+        hip.hipGraphExecDestroy(e)
+        hip.hipGraphDestroy(g)
+    for s in streams:
+        hip.hipStreamDestroy(s)

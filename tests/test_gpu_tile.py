@@ -72,10 +72,12 @@ def test_wide_linears_equal_oracle(group, bits, m, n):
     assert_equals_oracle(y, x, m, L, [(0, 130), (n // 2, n // 2 + 130), (n - 130, n)])
 
 
-@pytest.mark.parametrize("group,bits,m,n,k", [(128, 3, 40, 7000, 1024), (128, 2, 100, 600, 9344), (64, 4, 3, 600, 2112)])
+@pytest.mark.parametrize("group,bits,m,n,k", [(128, 3, 40, 7000, 1024), (128, 2, 100, 600, 9344), (64, 4, 3, 600, 2112),
+                                              (128, 2, 128, 40, 163840)])
 def test_equals_the_other_kernels(group, bits, m, n, k):
-    """The kernels an explicit crossover selects, the entry point without allocation, and a stream that has no scratch
-    when it is captured: the same bits; the captured launches replay."""
+    """The kernels an explicit crossover selects, the entry point without allocation (the last case's converted
+    activations are larger than its array: the older kernels), and captures of a stream that the library has not worked
+    on and has: the same bits; the captured launches, which are the tiled kernel's two, replay."""
     K = kernels()
     hip = ctypes.CDLL("libamdhip64.so")
     vp = ctypes.c_void_p
@@ -102,7 +104,7 @@ def test_equals_the_other_kernels(group, bits, m, n, k):
     assert np.array_equal(out(lambda Y: check(K.ak_wq_gemv_kt_multi_noalloc(*args(Y), None))), want)
     stream = vp()
     assert hip.hipStreamCreate(ctypes.byref(stream)) == 0
-    for warm in (False, True):  # without scratch, with it
+    for warm in (False, True):
         Y, graph, exe = Dev(m * n * 2), vp(), vp()
         if warm:
             check(K.ak_wq_gemv_kt_multi(*args(Y), stream))
@@ -111,6 +113,8 @@ def test_equals_the_other_kernels(group, bits, m, n, k):
         rc = K.ak_wq_gemv_kt_multi(*args(Y), stream)
         assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
         check(rc, "under capture")
+        count = ctypes.c_size_t()
+        assert hip.hipGraphGetNodes(graph, None, ctypes.byref(count)) == 0 and count.value == 2
         assert hip.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, ctypes.c_size_t(0)) == 0
         for rep in range(3):
             junk = np.full(m * n, 0x7FC1, dtype=np.uint16)
