@@ -52,8 +52,10 @@ __device__ __forceinline__ void own_row(u32x4& a, u32x4& b, bool odd) {
   }
 }
 
-// TT token tiles of 16 (m <= 16 TT), RB row blocks of 16 per workgroup, KU steps per group of requests
-template <int TT, int RB, int KU>
+// TT token tiles of 16 (m <= 16 TT), RB row blocks of 16 per workgroup, KU steps per group of requests.  WIDE: rows of
+// 2^24 inputs or more, which the buffers' 32-bit offsets do not cover: the same loads by address, at clamped rows, tokens
+// and inputs in place of zeros (what they hold is not used)
+template <int TT, int RB, int KU, bool WIDE = false>
 __global__ void __launch_bounds__(NW * 64) bi_gemv_kernel(const uint16_t* __restrict__ x, int m,
                                                               const uint16_t* __restrict__ w,
                                                               const uint16_t* __restrict__ bias,
@@ -63,7 +65,7 @@ __global__ void __launch_bounds__(NW * 64) bi_gemv_kernel(const uint16_t* __rest
   const int c = lane & 15, h = lane >> 4;
   const bool odd = c & 1;
   const int row0 = (int)blockIdx.x * 16 * RB;
-  const int steps = (k + 63) >> 6, s_lo = wave * steps / NW, s_hi = (wave + 1) * steps / NW;
+  const int steps = (int)(((unsigned)k + 63) >> 6), s_lo = wave * steps / NW, s_hi = (wave + 1) * steps / NW;
   // bytes of a lane's two loads within a step: the half line (c & 1), chunk h of it
   const unsigned lo = 64 * (c & 1) + 16 * h, k2 = 2u * k;
   const int nr = n - row0 < 16 * RB ? n - row0 : 16 * RB;
@@ -83,6 +85,21 @@ __global__ void __launch_bounds__(NW * 64) bi_gemv_kernel(const uint16_t* __rest
   // a step's loads; rows past n and tokens past m read zeros (out of the buffers' range), steps past the wave's last
   // are not used and mostly out of range too
   auto load = [&](int s, Step& d) __attribute__((always_inline)) {
+    if constexpr (WIDE) {
+      const int i = s < s_hi ? 64 * s + 32 * (c & 1) + 8 * h : 0, i1 = (unsigned)i < (unsigned)k ? i : 0;
+      auto at = [&](const uint16_t* p, int r, int rows) {
+        return __builtin_nontemporal_load(
+            reinterpret_cast<const u32x4*>(p + (size_t)(r < rows ? r : rows - 1) * k + i1));
+      };
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+#pragma unroll
+        for (int r = 0; r < RB; ++r) d.a[r][e] = at(w, row0 + 16 * r + (c & ~1) + e, n);
+#pragma unroll
+        for (int t = 0; t < TT; ++t) d.b[t][e] = at(x, 16 * t + (c & ~1) + e, m);
+      }
+      return;
+    }
     const unsigned v = v0 + (s < s_hi ? 128u * s : 0x40000000u);
 #pragma unroll
     for (int r = 0; r < RB; ++r)
@@ -95,7 +112,7 @@ __global__ void __launch_bounds__(NW * 64) bi_gemv_kernel(const uint16_t* __rest
   };
   auto use = [&](int s, Step& d) __attribute__((always_inline)) {
     if (s >= s_hi) return;
-    const bool cut = 64 * s + 32 >= k;
+    const bool cut = 64u * s + 32 >= (unsigned)k;
     const u32x4 z = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int r = 0; r < RB; ++r) {
@@ -176,10 +193,10 @@ __global__ void __launch_bounds__(NW * 64) bi_gemv_kernel(const uint16_t* __rest
   }
 }
 
-template <int TT, int RB, int KU>
+template <int TT, int RB, int KU, bool WIDE = false>
 void launch_bi(const uint16_t* x, int m, const uint16_t* w, const uint16_t* bias, uint16_t* y, int n, int k, long ldy,
                hipStream_t s) {
-  hipLaunchKernelGGL((bi_gemv_kernel<TT, RB, KU>), dim3((n + 16 * RB - 1) / (16 * RB)), dim3(NW * 64),
+  hipLaunchKernelGGL((bi_gemv_kernel<TT, RB, KU, WIDE>), dim3((n + 16 * RB - 1) / (16 * RB)), dim3(NW * 64),
                      NW * RB * TT * 64 * sizeof(f32x4), s, x, m, w, bias, y, n, k, ldy);
 }
 
@@ -193,14 +210,15 @@ int rows_per_workgroup(int n, int k, int m) {
   const double r = m <= 16 ? 1.5 : m <= 32 ? 1.4 : m <= 64 ? 1.33 : 1.2, bytes = 2.0 * n * k;
   const int nb = (n + 15) / 16, cus = num_cus();
   const double one = (nb + cus - 1) / cus * u, two = (nb + 2 * cus - 1) / (2 * cus) * r * u;
-  if (k >= 1 << 24) return 1;  // 32-bit buffer offsets
   return std::max(two, bytes / 6.0e6) < std::max(one, bytes / 7.3e6) ? 2 : 1;
 }
 
 template <int TT, int KU1, int KU2>
 void launch_rows(const uint16_t* x, int m, const uint16_t* w, const uint16_t* bias, uint16_t* y, int n, int k, long ldy,
                  hipStream_t s) {
-  if (rows_per_workgroup(n, k, m) == 2)
+  if (k >= 1 << 24)  // (128 tokens or 32 rows of fewer inputs stay within 32-bit buffer offsets)
+    launch_bi<TT, 1, KU1, true>(x, m, w, bias, y, n, k, ldy, s);
+  else if (rows_per_workgroup(n, k, m) == 2)
     launch_bi<TT, 2, KU2>(x, m, w, bias, y, n, k, ldy, s);
   else
     launch_bi<TT, 1, KU1>(x, m, w, bias, y, n, k, ldy, s);
@@ -219,21 +237,12 @@ extern "C" int ak_bf16_gemv_bi_ld(const void* x, const void* w, const void* bias
   auto W = static_cast<const uint16_t*>(w);
   auto B = static_cast<const uint16_t*>(bias);
   auto Y = static_cast<uint16_t*>(y);
-  // 32-bit buffer offsets: as many tokens per launch as they cover (all of them below k = 2^24)
-  if (k >= 1 << 27) return AK_INVALID;
-  const int most = k < 1 << 24 ? 128 : 16;
-  for (int m0 = 0; m0 < m; m0 += most) {
-    const int mm = m - m0 < most ? m - m0 : most;
-    const uint16_t* x0 = X + (size_t)m0 * k;
-    uint16_t* y0 = Y + (size_t)m0 * ldy;
-    const int tt = (mm + 15) / 16;
-    switch (tt) {
-      case 1: agq::launch_rows<1, 2, 2>(x0, mm, W, B, y0, n, k, ldy, s); break;
-      case 2: agq::launch_rows<2, 2, 2>(x0, mm, W, B, y0, n, k, ldy, s); break;
-      case 3:
-      case 4: agq::launch_rows<4, 1, 1>(x0, mm, W, B, y0, n, k, ldy, s); break;
-      default: agq::launch_rows<8, 1, 1>(x0, mm, W, B, y0, n, k, ldy, s); break;
-    }
+  switch ((m + 15) / 16) {
+    case 1: agq::launch_rows<1, 2, 2>(X, m, W, B, Y, n, k, ldy, s); break;
+    case 2: agq::launch_rows<2, 2, 2>(X, m, W, B, Y, n, k, ldy, s); break;
+    case 3:
+    case 4: agq::launch_rows<4, 1, 1>(X, m, W, B, Y, n, k, ldy, s); break;
+    default: agq::launch_rows<8, 1, 1>(X, m, W, B, Y, n, k, ldy, s); break;
   }
   return (int)hipGetLastError();
 }

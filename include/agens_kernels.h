@@ -171,7 +171,7 @@ int ak_i8_gemv(const void* x, const void* w, const void* scale, void* y, int m, 
 
 /* ---------------------------------------------------------------------------------------------- batch-invariant bf16 GEMV
  * y[t][r] (row stride ldy; n for ak_bf16_gemv_bi) = bf16(sum_i x[t][i] W[r][i] (+ bias[r])); W bf16 [n][k] row-major,
- * x bf16 [m][k], bias bf16 [n] or NULL; 1 <= m <= 128, k % 32 == 0, k < 2^27 (else 1).  fp32 accumulation (MFMA), the bias added
+ * x bf16 [m][k], bias bf16 [n] or NULL; 1 <= m <= 128, k % 32 == 0 (else 1).  fp32 accumulation (MFMA), the bias added
  * in fp32 before the one bf16 rounding, and a summation order that does not depend on m: row t of an m-token call is
  * bit-identical to the 1-token call.  The reference's bits come from its tensor-core MMA's internal accumulation, so
  * results agree with the reference within fp32-accumulation tolerance, not bit for bit. */

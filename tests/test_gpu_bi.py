@@ -86,3 +86,20 @@ def test_rows_bit_identical_for_every_m_and_ldy():
         assert np.array_equal(part, full[:m, :n]), f"m = {m}"
     one = run(x[77 * k: 78 * k], w, b, 1, n, k)
     assert np.array_equal(one, full[77, :n])
+
+
+# rows of 2^24 inputs and more (loads by address, not by 32-bit offset): row and token tiles with one and more entries, a
+# last half step, and the row length from which one row block exceeds 4 GB
+@pytest.mark.parametrize("m,n,k", [(1, 2, (1 << 24) - 32), (3, 1, 1 << 24), (17, 2, (1 << 24) + 96), (1, 1, 1 << 27),
+                                   (2, 1, (1 << 27) + 32)])
+def test_long_rows(m, n, k):
+    """Small integers: |sum| < 2^24 of every part of the order, so each output is the exact sum's one rounding."""
+    rng = np.random.default_rng(m + n + k)
+    xi, wi = (rng.integers(-2, 3, size=(r, k), dtype=np.int8) for r in (m, n))
+    table = f2bf_array(np.arange(-2, 3, dtype=np.float32))
+    got = run(table[(xi + 2).ravel()], table[(wi + 2).ravel()], None, m, n, k).reshape(m, n)
+    S = np.array([[sum(int(np.dot(x[i:i + (1 << 20)].astype(np.int32), w[i:i + (1 << 20)].astype(np.int32)))
+                       for i in range(0, k, 1 << 20)) for w in wi] for x in xi], dtype=np.float32)
+    assert np.abs(S).max() < 2 ** 22  # a random walk of steps below 4
+    want = f2bf_array(S.ravel()).reshape(m, n)
+    assert np.array_equal(got, want), (got, want)
