@@ -262,7 +262,6 @@ void launch_lds_rows(const uint16_t* x, const int8_t* w, const float* scale, uin
 void lds_part(const uint16_t* x, const int8_t* w, const float* scale, uint16_t* y, int m, int n, int k, int ldy,
               hipStream_t s) {
   switch (m) {
-    case 1: return launch_lds_rows<1>(x, w, scale, y, n, k, ldy, s);
     case 2: return launch_lds_rows<2>(x, w, scale, y, n, k, ldy, s);
     case 3: return launch_lds_rows<3>(x, w, scale, y, n, k, ldy, s);
     case 4: return launch_lds_rows<4>(x, w, scale, y, n, k, ldy, s);
@@ -287,12 +286,16 @@ extern "C" int ak_i8_gemv(const void* x, const void* w, const void* scale, void*
   auto Y = static_cast<uint16_t*>(y);
   auto wgs = [n](int rows) { return dim3((n + 8 * rows - 1) / (8 * rows)); };  // 8 half-waves per workgroup
   // Two to 16 tokens in parts of at most 8 whose activations take at most 80 KB of LDS (two workgroups per CU): the LDS
-  // kernel where at most two parts, i.e. two passes over the weights, cover them.  Measured (us, 152064 x 5120, before =
-  // activations from L1 per token and row pair): 2 / 4 / 8 / 16 tokens 156 / 233 / 358 / 628 -> 119 / 148 / 228 / 460.
-  // Two or three tokens on less than 32 MB of weights stay with the kernel below (8001 x 1040: 7.1 against 7.4, 7.4
-  // against 7.7).
-  const int cap = 81920 / (2 * k), most = cap < 8 ? cap : 8;
-  if (m > 1 && most > 0 && m <= 2 * most && (m > 3 || (long long)n * k >= 32 << 20)) {
+  // kernel where one part covers them, or two.  Measured (us, 152064 x 5120, before = activations from L1 per token and
+  // row pair): 2 / 4 / 8 / 16 tokens 156 / 233 / 358 / 628 -> 119 / 148 / 228 / 460.  Two or three tokens on less than 32
+  // MB of weights stay with the kernel below (8001 x 1040: 7.1 against 7.4, 7.4 against 7.7).
+  // The second part reads all weights again.  Below 32 MB they are still in the caches (1700 x 16400, 4 tokens 50.9 ->
+  // 44.2; 1700 x 13648, 6 tokens 55.5 -> 41.8); above, it pays only for parts of up to four tokens or more (60000 x 10240,
+  // 8 tokens 294 -> 267; 33000 x 8192, 9 tokens 176 -> 136), not for less (12000 x 24576, 2 tokens 73 against 104; 12000 x
+  // 16400, 4 tokens 78 against 97; 60000 x 12288, 6 tokens 319 against 338).
+  const int cap = 40960 / k, most = cap < 8 ? cap : 8;
+  const bool small = (long long)n * k < 32 << 20;
+  if (most > 0 && (small ? m > 3 && m <= 2 * most : m > 1 && m <= (most < 4 ? most : 2 * most))) {
     const int parts = (m + most - 1) / most, per = (m + parts - 1) / parts;
     for (int m0 = 0; m0 < m; m0 += per)
       agq::lds_part(X + (size_t)m0 * k, W, S, Y + (size_t)m0 * ldy, m - m0 < per ? m - m0 : per, n, k, ldy, s);
