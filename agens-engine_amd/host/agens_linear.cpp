@@ -125,8 +125,17 @@ int g_prefill_route = -1;  // -1: by shape, 0: dequantized tiles x library GEMM,
 //   qkv W4 7168 x 5120:       512:  60 vs  73,  768:  77 vs 103,   1024:  94 vs 113,   1280: 114 vs 97.
 // The fused kernel wins on every linear up to 768 tokens, on the widest up to 1024 and on long k up to 1536; the
 // library GEMM beyond (the fused kernel expands every weight once per token tile).
-bool prefill_fused(int n, int k, int m) {
+// It takes weights and activations below 2 GB each (32-bit buffer offsets).
+bool fused_fits(const QuantLinear& t, int m) {
+  const long long limit = 1ll << 31;
+  for (int j = 0; j < t.np; ++j)
+    if ((long long)ak_wq_kt_weight_bytes(t.p[j].bits, t.p[j].n, t.k) >= limit) return false;
+  return (long long)m * t.k * 2 < limit;
+}
+bool prefill_fused(const QuantLinear& t, int m) {
   if (g_prefill_route >= 0) return g_prefill_route == 1;
+  const int n = t.n, k = t.k;
+  if (!fused_fits(t, m)) return false;
   return m <= 768 || (k >= 16384 && m <= 1536) || (n >= 100000 && m <= 1024);
 }
 }  // namespace
@@ -135,7 +144,7 @@ void set_prefill_route(int mode) { g_prefill_route = mode < 0 ? -1 : (mode ? 1 :
 
 int linear(const QuantLinear& t, const void* x, void* y, int m, int n, int k, int bf16w, void* stream) {
   if (t.n != n || t.k != k || m < 1 || t.np < 1 || t.np > 2) return 1;
-  if (m > 128 && prefill_fused(n, k, m)) {
+  if (m > 128 && prefill_fused(t, m)) {
     // prefill through the fused GEMM: one launch per part, straight from the KT weights into its columns of y
     for (int j = 0; j < t.np; ++j) {
       const QuantPart& q = t.p[j];
