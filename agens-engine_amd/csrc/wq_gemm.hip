@@ -37,6 +37,7 @@
 #include <type_traits>
 
 #include "agens_kernels.h"
+#include "agens_tuning.h"
 #include "wq_common.h"
 
 
@@ -392,10 +393,12 @@ int launch_tiles(const void* x, int m, const void* wt, const void* st, void* y, 
 // tile that does not pad too many tokens, and narrow or short ones split k until one round is nearly full.  Measured
 // (us, T x splits): down 5120 x 27648 W2 at 333 tokens 192 x 6 112, 128 x 4 126, 256 x 6 130; at 256 tokens 128 x 6 91,
 // 128 x 8 119 (a second round); at 64 tokens 64 x 12 40, 64 x 8 49, 64 x 16 46; o 5120 x 5120 W4 at 256 tokens
-// 128 x 6 30, 128 x 4 34, 128 x 8 39.
+// 128 x 6 30, 128 x 4 34, 128 x 8 39.  Splits whose partials exceed kMaxCallScratch (four rounds of 256-token tiles) are
+// left out: down at 4096 tokens takes 256 x 3, not 256 x 4.
 struct Tiling {
   int T, split;
 };
+size_t part_bytes(long long tiles, int T, int split) { return (size_t)(tiles * split) * 1024 * T; }
 Tiling pick_tiling(int m, int n, int nslab, bool may_split) {
   const int xcd_cus = num_cus() / 8 > 0 ? num_cus() / 8 : 1;
   Tiling best = {256, 1};
@@ -404,6 +407,7 @@ Tiling pick_tiling(int m, int n, int nslab, bool may_split) {
     const double slab = T == 256 ? 1.75 : T == 192 ? 1.42 : T == 128 ? 1.12 : 0.78;
     const long long tiles = (long long)((n + 255) / 256) * ((m + T - 1) / T);
     for (int sp = 1; sp <= (may_split ? 32 : 1) && (sp == 1 || nslab / sp >= 4); ++sp) {
+      if (sp > 1 && part_bytes(tiles, T, sp) > kMaxCallScratch) break;
       const long long items = tiles * sp, rounds = ((items + 7) / 8 + xcd_cus - 1) / xcd_cus;
       const double us = (double)rounds * ((nslab + sp - 1) / sp * slab + 3.0) +
                         (sp > 1 ? 4.0 + 2048.0 * (double)items * T / 8e6 : 0.0);
@@ -431,8 +435,8 @@ int launch_gemm(const void* x, int m, const void* wt, const void* st, void* y, i
   std::unique_lock<std::mutex> lock;
   if (tl.split > 1) {
     lock = std::unique_lock<std::mutex>(scratch_mutex(s));  // the two kernels of a split launch stay together
-    part = reinterpret_cast<float*>(
-        call_scratch(s, (size_t)tl.split * ((n + 255) / 256) * ((m + tl.T - 1) / tl.T) * 1024 * tl.T).data);
+    const long long tiles = (long long)((n + 255) / 256) * ((m + tl.T - 1) / tl.T);
+    part = reinterpret_cast<float*>(call_scratch(s, part_bytes(tiles, tl.T, tl.split)).data);
     if (!part) tl = pick_tiling(m, n, k / kSlab, false);
   }
   switch (tl.T) {
@@ -445,6 +449,14 @@ int launch_gemm(const void* x, int m, const void* wt, const void* st, void* y, i
 
 }  // namespace
 }  // namespace agq
+
+extern "C" int ak_wq_gemm_tune_query(int m, int n, int k, int* tokens, int* splits, size_t* scratch) {
+  if (!tokens || !splits || !scratch || m < 1 || n < 1 || k < 64 || k % 64 != 0) return AK_INVALID;
+  const agq::Tiling t = agq::pick_tiling(m, n, k / agq::kSlab, true);
+  *tokens = t.T, *splits = t.split;
+  *scratch = t.split > 1 ? agq::part_bytes((long long)((n + 255) / 256) * ((m + t.T - 1) / t.T), t.T, t.split) : 0;
+  return 0;
+}
 
 // No single counterpart in the reference: the fusion of ak_wq_dequant_kt_rows (kernels/src/w4_gemv.cu:877-895) and
 // ak_bf16_linear_f32reduce_ld (kernels/src/bf16_linear.cu:68-80), the pair the model's linear() runs above 128 tokens

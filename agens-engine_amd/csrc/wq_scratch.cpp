@@ -134,10 +134,11 @@ void* stream_scratch(hipStream_t s, size_t bytes) {
       P.idle.erase(P.idle.begin() + (long)i);
       return replace_with(n);
     }
-  // at least double: a replaced buffer is kept, not freed (a graph captured before the growth still addresses it), so
-  // the replaced buffers stay below the current one in total
+  // at least double, up to the most that a call asks for: a replaced buffer is kept, not freed (a graph captured before
+  // the growth still addresses it), so the replaced buffers stay below twice the current one in total
   size_t want = bytes > ((size_t)4 << 20) ? bytes : ((size_t)4 << 20);
-  if (b.p && want < 2 * b.bytes) want = 2 * b.bytes;
+  const size_t twice = 2 * b.bytes < kMaxCallScratch + kCounters ? 2 * b.bytes : kMaxCallScratch + kCounters;
+  if (b.p && want < twice) want = twice;
   void* p = nullptr;
   if (hipMalloc(&p, want) != hipSuccess || hipMemset(p, 0, want) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
     if (p) (void)hipFree(p);

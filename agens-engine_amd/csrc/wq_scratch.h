@@ -24,6 +24,9 @@ std::mutex& scratch_mutex(hipStream_t s);
 // The scratch of stream s on the current device, at least `bytes` long; null without it (see wq_scratch.cpp).
 void* stream_scratch(hipStream_t s, size_t bytes);
 
+// The most data that one call asks of call_scratch: the launch shapes that need more are not considered
+constexpr size_t kMaxCallScratch = (size_t)256 << 20;
+
 // The same for a call that may be captured: 4 KB of counters (zero between launches) and `bytes` of data that no other
 // stream and no other graph works in; null pointers without it.
 struct CallScratch {

@@ -69,8 +69,7 @@ int tile_gemv(int bits, const void* x, int m, const Segs& g, int k, int group, h
   size_t part = 0;
   if (t.sk)
     for (int i = 0; i < g.nseg; ++i) part += (size_t)a.P * a.ntt * ((g.n[i] + 15) / 16) * 1024;
-  constexpr size_t kMaxScratch = (size_t)256 << 20;  // (128 tokens x 27648 inputs x 5120 rows: 33 MB)
-  if (4096 + part + a.img_bytes > kMaxScratch) return AK_INVALID;
+  if (part + a.img_bytes > kMaxCallScratch) return AK_INVALID;  // (128 tokens x 27648 inputs x 5120 rows: 33 MB)
   const CallScratch z = call_scratch(s, part + a.img_bytes);
   if (!z.data) return AK_INVALID;
   a.cnt = z.cnt;

@@ -141,3 +141,20 @@ def test_launch_table_pins_are_honoured(K):
     K.ak_wq_tune_override(0, 0, -1)
     assert K.ak_wq_tune_query(3, 1, 1, ns, 5120, *[ctypes.byref(g) for g in got]) == 0
     assert tuple(g.value for g in got) == before
+
+
+def test_prefill_gemm_scratch_is_bounded(K):
+    """The partial sums of a k-split prefill GEMM stay within 256 MiB at every shape, and are what the tiling says."""
+    T, S, B = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t()
+    split = 0
+    for m in (1, 129, 333, 512, 1024, 2048, 4030, 4096, 8192, 16384, 65536):
+        for n, k in ((1, 64), (1024, 5120), (5120, 5120), (5120, 27648), (7168, 5120), (13507, 18048), (55296, 5120),
+                     (152064, 5120), (2048, 65536)):
+            assert K.ak_wq_gemm_tune_query(m, n, k, ctypes.byref(T), ctypes.byref(S), ctypes.byref(B)) == 0
+            tiles = -(-n // 256) * -(-m // T.value)
+            assert T.value in (64, 128, 192, 256) and 1 <= S.value <= 32
+            assert B.value == (tiles * S.value * T.value * 1024 if S.value > 1 else 0)
+            assert B.value <= 256 << 20, (m, n, k, T.value, S.value, B.value)
+            split += S.value > 1
+    assert split > 10
+    assert K.ak_wq_gemm_tune_query(0, 1, 64, ctypes.byref(T), ctypes.byref(S), ctypes.byref(B)) == 1
