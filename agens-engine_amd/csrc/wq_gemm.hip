@@ -4,14 +4,14 @@
 // The reference's prefill route (kernels/m1/m1_model.cu:1876-1897) dequantizes a tile of output rows into a bf16
 // scratch (2 bytes per weight written, then read again) and runs a library GEMM (ak_bf16_linear_f32reduce_ld,
 // kernels/src/bf16_linear.cu:68-92).  Here the KT records are read once per token tile, expanded to bf16 in registers
-// and written to LDS, and v_mfma_f32_16x16x32_bf16 consumes them there: no dequantized copy, no second pass over the
-// weights (narrow linears split k across workgroups, with fp32 partials in the stream's split-K scratch).
+// and written to LDS, and v_mfma_f32_32x32x16_bf16 consumes them there: no dequantized copy, no second pass over the
+// weights (narrow linears split k across workgroups, with fp32 partials in call_scratch).
 //
-// Tiling: 256 output rows x T tokens (T = 64, 128, 192, 256, by pick_tiling) per workgroup of 8 waves, wave tiles of 64
-// rows x T / 2 tokens as 32 x 32 MFMA tiles, k in slabs of 64 inputs.  Thread (row tid / 2, half tid % 2) loads its lane
+// Tiling: R = 256 output rows x T tokens (T = 64, 128, 192, 256) per workgroup of 8 waves, or 128 x 128 per workgroup of 4
+// (by pick_tiling), wave tiles of 64 rows x T / 2 tokens as 32 x 32 MFMA tiles, k in slabs of 64 inputs.  Thread (row tid / 2, half tid % 2) loads its lane
 // chunk of the slab from the row's KT record (W4 16 B, W3 8 + 4 B, W2 8 B) and the group's scale three slabs ahead into
 // one of two register sets; the tokens go straight from the buffer into LDS (buffer loads into LDS, two stages, two
-// slabs ahead); the weights are dequantized once per T tokens into two 32 KB LDS stages.
+// slabs ahead); the weights are dequantized once per T tokens into two LDS stages (32 KB at R = 256).
 // What bounds it: per slab a SIMD's two waves need 2048 cycles of MFMA at T = 256, the workgroup's operand reads and
 // writes the LDS for as long, and the dequantization about 1400 cycles of each SIMD's VALU; each is hidden behind the
 // others only if no wave waits for its own.  So the slab is pipelined in slices of 16 inputs: the operands of a slice (24
@@ -23,6 +23,8 @@
 // Measured (us, before = 16 x 16 MFMA tiles with each slice's operands read right before its MFMAs): gate_up 55296 x
 // 5120 W3 at 512 tokens 334 -> 283, 300 tokens 326 -> 229 (T = 192), 2048 tokens 1172 -> 1049; o 5120 x 5120 W4 at 256
 // tokens 41 -> 31; down 5120 x 27648 W2 at 333 tokens 162 -> 112; 1.0-1.1 PFLOP/s where a round of tiles is full.
+// Few tiles (R = 256 only -> with the small tile): 2000 x 1024 W4 at 512 tokens 19.2 -> 13.7, 1000 x 4096 W3 at 512 23.0
+// -> 21.3, 3000 x 2048 W2 at 512 28.1 -> 23.8, 14000 x 1024 W3 at 64 19.6 -> 14.2.
 // Grid: the items (split, token tile, row tile) in that order cut into 8 contiguous runs, XCD x (workgroup i runs on XCD
 // i % 8) taking run x, so that each XCD works on one or two token tiles (T tokens x k inputs) that stay in its L2 while
 // the weights stream, and every XCD has as many workgroups as the others.
@@ -39,8 +41,6 @@
 #include "agens_kernels.h"
 #include "agens_tuning.h"
 #include "wq_common.h"
-
-
 
 namespace agq {
 int num_cus();
@@ -143,14 +143,15 @@ __device__ __forceinline__ u32x4 dequant_half(const HalfCodes& c, float s, int s
 }
 
 // SPLIT: k is split across workgroups; an item's fp32 tile goes to part[item] as its waves hold it (sum_splits_kernel)
-template <int BITS, int G, int T, bool SPLIT>
-__global__ void __launch_bounds__(512, T == 64 ? 4 : 1) wq_gemm_kernel(const uint16_t* __restrict__ x, int m,
+template <int BITS, int G, int R, int T, bool SPLIT>
+__global__ void __launch_bounds__(2 * R, R == 128 ? 2 : T == 64 ? 4 : 1) wq_gemm_kernel(const uint16_t* __restrict__ x, int m,
                                                               const uint8_t* __restrict__ wt,
                                                               const uint16_t* __restrict__ st,
                                                               uint16_t* __restrict__ y, int n, int ldy, int k,
                                                               int nrow_tiles, int ntok_tiles, int nsplit,
                                                               float* __restrict__ part) {
-  constexpr int R = 256, NJ = T / 64, XPW = T / 64;  // 32-token tiles per wave, 1 KB token blocks per wave and slab
+  constexpr int NW = R / 32, RW = R / 64;             // waves, along the rows
+  constexpr int NJ = T / 64, XPW = T / (8 * NW);      // 32-token tiles per wave, 1 KB token blocks per wave and slab
   constexpr int kWStage = R * kRowBytes, kXStage = T * kRowBytes, kXBase = 2 * kWStage;
   constexpr int OFF = BITS == 4 ? 8 : BITS == 3 ? 4 : 2;
   constexpr int REC = 128 * BITS, CB = BITS == 4 ? 16 : 8;
@@ -197,7 +198,7 @@ __global__ void __launch_bounds__(512, T == 64 ? 4 : 1) wq_gemm_kernel(const uin
     sl = sb + (sl < nslab ? sl : nslab - 1);
 #pragma unroll
     for (int j = 0; j < XPW; ++j)
-      lds_dma16(rx, lds + kXBase + xs * kXStage + (wave + 8 * j) * 1024, vx + j * 64 * k * 2, sl * kSlab * 2);
+      lds_dma16(rx, lds + kXBase + xs * kXStage + (wave + NW * j) * 1024, vx + j * 8 * NW * k * 2, sl * kSlab * 2);
   };
   // word u (8 inputs) of the thread's chunk, dequantized into weight stage `stage`
   auto put = [&](const ChunkRaw<BITS>& d, int u, int stage) __attribute__((always_inline)) {
@@ -209,7 +210,7 @@ __global__ void __launch_bounds__(512, T == 64 ? 4 : 1) wq_gemm_kernel(const uin
       *reinterpret_cast<u32x4*>(dst) = dequant_half<OFF>(half_codes<BITS>(d, u >> 1), sc, u & 1);
   };
 
-  const int wr = (wave & 3) * 64, wtk = (wave >> 2) * (T / 2);
+  const int wr = (wave % RW) * 64, wtk = (wave / RW) * (T / 2);
   const int l32 = lane & 31, hi = lane >> 5;
   f32x16 acc[2][NJ];
 #pragma unroll
@@ -313,7 +314,7 @@ __global__ void __launch_bounds__(512, T == 64 ? 4 : 1) wq_gemm_kernel(const uin
       for (int g = 0; g < 4; ++g) {
         const int r0 = o0 + wr + 32 * i + 8 * g + 4 * hi;
         if constexpr (SPLIT) {
-          reinterpret_cast<f32x4*>(part)[((size_t)item * (64 * NJ) + ((wave * NJ + j) * 2 + i) * 4 + g) * 64 + lane] =
+          reinterpret_cast<f32x4*>(part)[((size_t)item * (8 * NW * NJ) + ((wave * NJ + j) * 2 + i) * 4 + g) * 64 + lane] =
               f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
         } else {
           uint16_t* yr = y + (size_t)t * ldy;
@@ -334,20 +335,22 @@ __global__ void __launch_bounds__(512, T == 64 ? 4 : 1) wq_gemm_kernel(const uin
 }
 
 // y = bf16 of the splits' partials added in order.  A split's partials of a tile lie as its waves hold them (16 bytes per
-// lane: 4 rows of one token; 64 NJ such kilobytes per tile), so that they are written and read in whole lines; a thread
-// sums one 16-byte piece.  Eight splits' loads are requested before their sums (splits past the last one read the last
+// lane: 4 rows of one token; R T / 256 such kilobytes per tile), so that they are written and read in whole lines; a
+// thread sums one 16-byte piece.  Eight splits' loads are requested before their sums (splits past the last one read the last
 // one again and are not added): one memory round trip per eight splits instead of one per split.
 __global__ void __launch_bounds__(256) sum_splits_kernel(const f32x4* __restrict__ part, int nsplit, int m, int n,
                                                          uint16_t* __restrict__ y, int ldy, int nrow_tiles, int tiles,
-                                                         int nj) {
+                                                         int R, int nj) {
   const int f = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;  // kilobyte of the tile, its lane
   const int tile = blockIdx.y, tt = tile / nrow_tiles, rt = tile - tt * nrow_tiles;
   const int wj = f >> 3, wave = wj / nj, j = wj - wave * nj;
-  const int t = (tt * 2 + (wave >> 2)) * 32 * nj + 32 * j + (lane & 31);
-  const int o = rt * 256 + (wave & 3) * 64 + 8 * (f & 7) + 4 * (lane >> 5);
+  const int rw = R >> 6, wt = wave / rw;  // waves along the rows; the wave along the tokens
+  const int t = (tt * 2 + wt) * 32 * nj + 32 * j + (lane & 31);
+  const int o = rt * R + (wave - wt * rw) * 64 + 8 * (f & 7) + 4 * (lane >> 5);
   if (t >= m || o >= n) return;
-  const f32x4* p = part + ((size_t)tile * (64 * nj) + f) * 64 + lane;
-  const size_t step = (size_t)tiles * (64 * nj) * 64;
+  const int kb = R * nj >> 2;  // kilobytes of a tile
+  const f32x4* p = part + ((size_t)tile * kb + f) * 64 + lane;
+  const size_t step = (size_t)tiles * kb * 64;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   for (int s0 = 0; s0 < nsplit; s0 += 8) {
     f32x4 v[8];
@@ -368,60 +371,65 @@ __global__ void __launch_bounds__(256) sum_splits_kernel(const f32x4* __restrict
   }
 }
 
-template <int BITS, int G, int T, bool SPLIT>
+template <int BITS, int G, int R, int T, bool SPLIT>
 int launch_tiles(const void* x, int m, const void* wt, const void* st, void* y, int n, int ldy, int k, hipStream_t s,
                 int nsplit = 1, float* part = nullptr) {
-  const int nrt = (n + 255) / 256, ntt = (m + T - 1) / T;
+  const int nrt = (n + R - 1) / R, ntt = (m + T - 1) / T;
   const long long grid = ((long long)nrt * ntt * nsplit + 7) / 8 * 8;
   if (grid > 0x7FFFFFFF) return AK_INVALID;
-  hipLaunchKernelGGL((wq_gemm_kernel<BITS, G, T, SPLIT>), dim3((unsigned)grid), dim3(512),
-                     2 * (256 + T) * kRowBytes, s, static_cast<const uint16_t*>(x), m,
+  hipLaunchKernelGGL((wq_gemm_kernel<BITS, G, R, T, SPLIT>), dim3((unsigned)grid), dim3(2 * R),
+                     2 * (R + T) * kRowBytes, s, static_cast<const uint16_t*>(x), m,
                      static_cast<const uint8_t*>(wt), static_cast<const uint16_t*>(st), static_cast<uint16_t*>(y), n,
                      ldy, k, nrt, ntt, nsplit, part);
   if (SPLIT)
-    hipLaunchKernelGGL(sum_splits_kernel, dim3(T / 4, (unsigned)(nrt * ntt)), dim3(256), 0, s,
+    hipLaunchKernelGGL(sum_splits_kernel, dim3(R * T / 1024, (unsigned)(nrt * ntt)), dim3(256), 0, s,
                        reinterpret_cast<const f32x4*>(part), nsplit, m, n, static_cast<uint16_t*>(y), ldy, nrt,
-                       nrt * ntt, T / 64);
+                       nrt * ntt, R, T / 64);
   return (int)hipGetLastError();
 }
 
 // The tiling of a launch: T tokens per tile and the number of k splits, by the estimated time
-//   rounds x (slabs x slab time(T) + 3) + (split: 4 + the fp32 partials written and read at 8 TB/s) us,
+//   rounds x (slabs x slab time(R, T) + 3) + (split: 5 + the fp32 partials written and read at 8 TB/s) us,
 // rounds = workgroups per XCD / CUs per XCD, rounded up (one workgroup per CU at a time: at T = 64 two fit, but share
-// the same throughput).  Slab times measured at 240 workgroups (us): 0.78 at 64 tokens, 1.12 at 128, 1.42 at 192, 1.75 at
-// 256 (the dequantization and the weight tile's LDS traffic do not shrink with T).  So wide linears take the largest
-// tile that does not pad too many tokens, and narrow or short ones split k until one round is nearly full.  Measured
+// the same throughput).  Slab times measured at 240 workgroups (us): 0.65 at 128 x 128, 0.78 at 256 rows x 64 tokens, 1.12
+// at 128, 1.42 at 192, 1.75 at 256 (the dequantization and the weight tile's LDS traffic do not shrink with T).  So wide
+// linears take the largest tile that does not pad too many tokens, and narrow or short ones the smallest, with k split
+// until one round is nearly full.  Measured
 // (us, T x splits): down 5120 x 27648 W2 at 333 tokens 192 x 6 112, 128 x 4 126, 256 x 6 130; at 256 tokens 128 x 6 91,
 // 128 x 8 119 (a second round); at 64 tokens 64 x 12 40, 64 x 8 49, 64 x 16 46; o 5120 x 5120 W4 at 256 tokens
 // 128 x 6 30, 128 x 4 34, 128 x 8 39.  Splits whose partials exceed kMaxCallScratch (four rounds of 256-token tiles) are
 // left out: down at 4096 tokens takes 256 x 3, not 256 x 4.
 struct Tiling {
-  int T, split;
+  int R, T, split;
 };
-size_t part_bytes(long long tiles, int T, int split) { return (size_t)(tiles * split) * 1024 * T; }
+long long tiles_of(const Tiling& t, int m, int n) { return (long long)((n + t.R - 1) / t.R) * ((m + t.T - 1) / t.T); }
+size_t part_bytes(const Tiling& t, int m, int n) { return (size_t)(tiles_of(t, m, n) * t.split) * 4 * t.R * t.T; }
 Tiling pick_tiling(int m, int n, int nslab, bool may_split) {
   const int xcd_cus = num_cus() / 8 > 0 ? num_cus() / 8 : 1;
-  Tiling best = {256, 1};
+  Tiling best = {256, 256, 1};
   double best_us = 1e30;
-  for (int T = 64; T <= 256; T += 64) {
-    const double slab = T == 256 ? 1.75 : T == 192 ? 1.42 : T == 128 ? 1.12 : 0.78;
-    const long long tiles = (long long)((n + 255) / 256) * ((m + T - 1) / T);
+  for (int c = 0; c < 5; ++c) {
+    static const struct {
+      int R, T;
+      double slab;
+    } kTiles[5] = {{128, 128, 0.65}, {256, 64, 0.78}, {256, 128, 1.12}, {256, 192, 1.42}, {256, 256, 1.75}};
     for (int sp = 1; sp <= (may_split ? 32 : 1) && (sp == 1 || nslab / sp >= 4); ++sp) {
-      if (sp > 1 && part_bytes(tiles, T, sp) > kMaxCallScratch) break;
-      const long long items = tiles * sp, rounds = ((items + 7) / 8 + xcd_cus - 1) / xcd_cus;
-      const double us = (double)rounds * ((nslab + sp - 1) / sp * slab + 3.0) +
-                        (sp > 1 ? 4.0 + 2048.0 * (double)items * T / 8e6 : 0.0);
-      if (us < best_us) best_us = us, best = {T, sp};
+      const Tiling t = {kTiles[c].R, kTiles[c].T, sp};
+      if (sp > 1 && part_bytes(t, m, n) > kMaxCallScratch) break;
+      const long long items = tiles_of(t, m, n) * sp, rounds = ((items + 7) / 8 + xcd_cus - 1) / xcd_cus;
+      const double us = (double)rounds * ((nslab + sp - 1) / sp * kTiles[c].slab + 3.0) +
+                        (sp > 1 ? 5.0 + 2.0 * part_bytes(t, m, n) / 8e6 : 0.0);
+      if (us < best_us) best_us = us, best = t;
     }
   }
   return best;
 }
 
-template <int BITS, int G, int T>
+template <int BITS, int G, int R, int T>
 int launch_t(const void* x, int m, const void* wt, const void* st, void* y, int n, int ldy, int k, hipStream_t s,
              int nsplit, float* part) {
-  return part ? launch_tiles<BITS, G, T, true>(x, m, wt, st, y, n, ldy, k, s, nsplit, part)
-              : launch_tiles<BITS, G, T, false>(x, m, wt, st, y, n, ldy, k, s);
+  return part ? launch_tiles<BITS, G, R, T, true>(x, m, wt, st, y, n, ldy, k, s, nsplit, part)
+              : launch_tiles<BITS, G, R, T, false>(x, m, wt, st, y, n, ldy, k, s);
 }
 
 template <int BITS, int G>
@@ -435,26 +443,26 @@ int launch_gemm(const void* x, int m, const void* wt, const void* st, void* y, i
   std::unique_lock<std::mutex> lock;
   if (tl.split > 1) {
     lock = std::unique_lock<std::mutex>(scratch_mutex(s));  // the two kernels of a split launch stay together
-    const long long tiles = (long long)((n + 255) / 256) * ((m + tl.T - 1) / tl.T);
-    part = reinterpret_cast<float*>(call_scratch(s, part_bytes(tiles, tl.T, tl.split)).data);
+    part = reinterpret_cast<float*>(call_scratch(s, part_bytes(tl, m, n)).data);
     if (!part) tl = pick_tiling(m, n, k / kSlab, false);
   }
+  if (tl.R == 128) return launch_t<BITS, G, 128, 128>(x, m, wt, st, y, n, ldy, k, s, tl.split, part);
   switch (tl.T) {
-    case 64: return launch_t<BITS, G, 64>(x, m, wt, st, y, n, ldy, k, s, tl.split, part);
-    case 128: return launch_t<BITS, G, 128>(x, m, wt, st, y, n, ldy, k, s, tl.split, part);
-    case 192: return launch_t<BITS, G, 192>(x, m, wt, st, y, n, ldy, k, s, tl.split, part);
-    default: return launch_t<BITS, G, 256>(x, m, wt, st, y, n, ldy, k, s, tl.split, part);
+    case 64: return launch_t<BITS, G, 256, 64>(x, m, wt, st, y, n, ldy, k, s, tl.split, part);
+    case 128: return launch_t<BITS, G, 256, 128>(x, m, wt, st, y, n, ldy, k, s, tl.split, part);
+    case 192: return launch_t<BITS, G, 256, 192>(x, m, wt, st, y, n, ldy, k, s, tl.split, part);
+    default: return launch_t<BITS, G, 256, 256>(x, m, wt, st, y, n, ldy, k, s, tl.split, part);
   }
 }
 
 }  // namespace
 }  // namespace agq
 
-extern "C" int ak_wq_gemm_tune_query(int m, int n, int k, int* tokens, int* splits, size_t* scratch) {
-  if (!tokens || !splits || !scratch || m < 1 || n < 1 || k < 64 || k % 64 != 0) return AK_INVALID;
+extern "C" int ak_wq_gemm_tune_query(int m, int n, int k, int* rows, int* tokens, int* splits, size_t* scratch) {
+  if (!rows || !tokens || !splits || !scratch || m < 1 || n < 1 || k < 64 || k % 64 != 0) return AK_INVALID;
   const agq::Tiling t = agq::pick_tiling(m, n, k / agq::kSlab, true);
-  *tokens = t.T, *splits = t.split;
-  *scratch = t.split > 1 ? agq::part_bytes((long long)((n + 255) / 256) * ((m + t.T - 1) / t.T), t.T, t.split) : 0;
+  *rows = t.R, *tokens = t.T, *splits = t.split;
+  *scratch = t.split > 1 ? agq::part_bytes(t, m, n) : 0;
   return 0;
 }
 

@@ -23,9 +23,9 @@ int ak_wq_tune_override(int split, int nwv, int sk);
  * applied): 0 and *split, *nwv, *sk (1: split-K across workgroups), or 1 if the shape is not one this kernel takes. */
 int ak_wq_tune_query(int bits, int m, int nseg, const int* n, int k, int* split, int* nwv, int* sk);
 
-/* The tiling of an ak_wq_gemm_kt call: tokens per tile, k splits (1: none) and the bytes of scratch that the splits'
- * partial sums take.  0, or 1 for a shape that the call refuses. */
-int ak_wq_gemm_tune_query(int m, int n, int k, int* tokens, int* splits, size_t* scratch);
+/* The tiling of an ak_wq_gemm_kt call: rows and tokens per tile, k splits (1: none) and the bytes of scratch that the
+ * splits' partial sums take.  0, or 1 for a shape that the call refuses. */
+int ak_wq_gemm_tune_query(int m, int n, int k, int* rows, int* tokens, int* splits, size_t* scratch);
 
 /* The smallest token count (m) that ak_wq_gemv_kt_multi and its conveniences route to the fp16-MFMA kernel in the
  * default numerics (group 128): m >= this many tokens take it, fewer take the integer-limb kernels, at every k.  0:

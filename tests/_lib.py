@@ -313,7 +313,7 @@ def kernels():
             "ak_wq_chain_status": (i, []),
             "ak_w4_set_mma": (i, [i]),
             "ak_wq_set_mm_min": (i, [i]),
-            "ak_wq_gemm_tune_query": (i, [i, i, i, vp, vp, vp]),
+            "ak_wq_gemm_tune_query": (i, [i, i, i, vp, vp, vp, vp]),
             "ak_w4_set_lean": (i, [i]),
             "ak_w4_set_tma": (i, [i]),
         }

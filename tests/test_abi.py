@@ -145,16 +145,17 @@ def test_launch_table_pins_are_honoured(K):
 
 def test_prefill_gemm_scratch_is_bounded(K):
     """The partial sums of a k-split prefill GEMM stay within 256 MiB at every shape, and are what the tiling says."""
-    T, S, B = ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t()
+    R, T, S, B = ctypes.c_int(), ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t()
+    out = [ctypes.byref(v) for v in (R, T, S, B)]
     split = 0
     for m in (1, 129, 333, 512, 1024, 2048, 4030, 4096, 8192, 16384, 65536):
         for n, k in ((1, 64), (1024, 5120), (5120, 5120), (5120, 27648), (7168, 5120), (13507, 18048), (55296, 5120),
                      (152064, 5120), (2048, 65536)):
-            assert K.ak_wq_gemm_tune_query(m, n, k, ctypes.byref(T), ctypes.byref(S), ctypes.byref(B)) == 0
-            tiles = -(-n // 256) * -(-m // T.value)
-            assert T.value in (64, 128, 192, 256) and 1 <= S.value <= 32
-            assert B.value == (tiles * S.value * T.value * 1024 if S.value > 1 else 0)
+            assert K.ak_wq_gemm_tune_query(m, n, k, *out) == 0
+            tiles = -(-n // R.value) * -(-m // T.value)
+            assert (R.value, T.value) in ((128, 128), (256, 64), (256, 128), (256, 192), (256, 256)) and 1 <= S.value <= 32
+            assert B.value == (tiles * S.value * R.value * T.value * 4 if S.value > 1 else 0)
             assert B.value <= 256 << 20, (m, n, k, T.value, S.value, B.value)
             split += S.value > 1
     assert split > 10
-    assert K.ak_wq_gemm_tune_query(0, 1, 64, ctypes.byref(T), ctypes.byref(S), ctypes.byref(B)) == 1
+    assert K.ak_wq_gemm_tune_query(0, 1, 64, *out) == 1

@@ -169,6 +169,22 @@ def test_gemm_tilings_exact_on_small_integer_operands(bits, group, m, n, k):
     assert (y[:, n:] == 0x7FC1).all()
 
 
+# (the tiling that the shape takes, rows x tokens, and whether k is split): the smaller tile at its edges, with few, odd
+# and many slabs, and the others split
+@pytest.mark.parametrize("bits,group,m,n,k,tile,split", [
+    (4, 64, 127, 1, 64, (128, 128), False), (3, 128, 129, 385, 128, (128, 128), False),
+    (2, 64, 130, 4097, 192, (128, 128), False), (4, 128, 1025, 1999, 128, (128, 128), False),
+    (3, 64, 383, 1023, 2112, (128, 128), True), (2, 128, 128, 129, 4096, (128, 128), True),
+    (4, 64, 33, 1000, 4160, (256, 64), True), (3, 64, 64, 2331, 4160, (256, 64), True),
+    (2, 64, 385, 5117, 4160, (256, 128), True), (4, 64, 129, 9999, 4160, (256, 192), True),
+    (3, 64, 385, 9999, 4160, (256, 256), True)])
+def test_gemm_every_tile_exact_on_small_integer_operands(bits, group, m, n, k, tile, split):
+    r, t, sp, nbytes = ctypes.c_int(), ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t()
+    assert kernels().ak_wq_gemm_tune_query(m, n, k, *[ctypes.byref(v) for v in (r, t, sp, nbytes)]) == 0
+    assert (r.value, t.value) == tile and (sp.value > 1) == split
+    test_gemm_tilings_exact_on_small_integer_operands(bits, group, m, n, k)
+
+
 def test_split_k_gemm_leaves_gemv_scratch_intact():
     """A narrow long-k GEMM splits k across workgroups (fp32 partials in the stream's scratch); the split-K GEMV
     launches on the same stream keep their row-range counters in the first 4 KB of that scratch, zero between
