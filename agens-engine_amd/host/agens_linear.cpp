@@ -124,7 +124,10 @@ int g_prefill_route = -1;  // -1: by shape, 0: dequantized tiles x library GEMM,
 //   o W4 5120 x 5120:         512:  48 vs  49,  768:  60 vs  67,   1024:  73 vs  67;
 //   qkv W4 7168 x 5120:       512:  60 vs  73,  768:  77 vs 103,   1024:  94 vs 113,   1280: 114 vs 97.
 // The fused kernel wins on every linear up to 768 tokens, on the widest up to 1024 and on long k up to 1536; the
-// library GEMM beyond (the fused kernel expands every weight once per token tile).
+// library GEMM beyond (the fused kernel expands every weight once per token tile), and from about 600 tokens on middling
+// rows of short k, where the fused kernel's tiles fill a second round to a small part:
+//   8192 x 3072: 512: 39 vs 41, 600: 56 vs 47, 640: 56 vs 45;  6144 x 2560: 640: 31 vs 35, 700: 43 vs 37;
+//   4096 x 4096: 640: 40 vs 39, 700: 44 vs 40;  but 8192 x 2048: 640: 36 vs 36;  8192 x 5120: 640: 80 vs 95.
 // It takes weights and activations below 2 GB each (32-bit buffer offsets).
 bool fused_fits(const QuantLinear& t, int m) {
   const long long limit = 1ll << 31;
@@ -136,6 +139,7 @@ bool prefill_fused(const QuantLinear& t, int m) {
   if (g_prefill_route >= 0) return g_prefill_route == 1;
   const int n = t.n, k = t.k;
   if (!fused_fits(t, m)) return false;
+  if (m > 576 && n >= 4096 && n <= 8192 && k > 2048 && k <= 4096) return false;
   return m <= 768 || (k >= 16384 && m <= 1536) || (n >= 100000 && m <= 1024);
 }
 }  // namespace

@@ -64,6 +64,10 @@ int main() {
   linear(4, 512, 5120, 5120, true, "fused up to 768 tokens");
   linear(4, 769, 5120, 5120, false, "the library GEMM above");
   linear(2, 1536, 5120, 27648, true, "fused up to 1536 tokens at long k");
+  linear(4, 577, 8192, 4096, false, "the library GEMM on middling rows of short k");
+  linear(4, 576, 8192, 4096, true, "fused up to 576 tokens there");
+  linear(4, 768, 8192, 2048, true, "and at shorter k");
+  linear(4, 768, 8193, 4096, true, "and on more rows");
   // weights of 2 GB and just below, activations of 2 GB and just below, at every route's token counts
   linear(4, 1100, 131072, 32768, false, "weights of 2 GB, long k");
   linear(4, 1100, 131071, 32768, true, "weights just below");
