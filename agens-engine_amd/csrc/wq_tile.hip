@@ -18,9 +18,12 @@ int row_ranges(const Segs& g, int blocks) {  // workgroups that cover the segmen
 // The launch shape with the smallest estimated time (rb = 0: none fits).  Workgroups run in rounds of one per CU; a step
 // (one group of inputs) takes about 0.45 + 0.21 rb us at group 128 and three quarters of that at group 64 (measured us
 // per step, g128: 0.65 at 1 block per wave, 0.85 at 2, 1.25 at 4, 1.5 at 5, 1.95 at 7; g64: 0.52 at 1, 0.7 at 2, 1.4 at
-// 7), two workgroups of up to 2 blocks per wave share a CU at about 0.85 of the time, and a split adds its partials'
-// traffic and the last workgroups' sums.  So wide linears run unsplit with the most blocks per wave that do not start
-// another round, narrow ones split k at the size that fills one (measured, us):
+// 7), two workgroups of up to 2 blocks per wave share a CU at about 0.85 of the time.  A split takes as long as its
+// longest stripe, and adds its partials' traffic (2 us per 4 MB, 2.5 at group 64) and the last workgroups' sums: 9 tiles
+// are 2 per stripe, not 9 / 8 (20000 x 8320 W2, 33 tokens: split 132, unsplit 87; 90000 x 9216 W4 g64, 1 token: 211 and
+// 140), and many rows pay more for the partials than for another round (98304 x 8192 W4 g64, 1 token: split 151, unsplit
+// 130).  So wide linears run unsplit with the most blocks per wave that do not start another round, narrow ones split k
+// at the size that fills one (measured, us):
 //   gate_up 55296 x 5120 W3, 64 tokens: 7 blocks (247 workgroups) 86, 5 (346) 132, 4 (432) 103;
 //   down 5120 x 27648 W2, 64 tokens, split: 5 blocks (256 workgroups) 60, 4 (320) 92, 2 (640) 88;
 //   o 5120 x 5120 W4, 64 tokens: split 4 blocks (200) 28.8, 2 (400) 32.2, unsplit 2 blocks (80) 35.1;
@@ -39,9 +42,9 @@ TileShape pick_shape(const TileArgs& a, int group) {
       const int ranges = row_ranges(a.segs, rg * t.rb);
       if (tile_lds(t, group, a.ntt) > 160 * 1024 || (sk && ranges > 1024)) continue;
       const long long rounds = ((long long)ranges * (sk ? a.P : 1) + cus - 1) / cus;
-      const double steps = (sk ? (double)ntile / a.P : (double)ntile) * (1024 / group);
+      const double steps = (sk ? (ntile + a.P - 1) / a.P : ntile) * (1024.0 / group);
       const double us = rounds * (t.rb <= 2 && rounds > 1 ? 0.85 : 1.0) * steps * (0.45 + 0.21 * t.rb) * (group == 64 ? 0.75 : 1.0) +
-                        (sk ? 4.0 + 2.0 * 1024 / 4e6 * a.P * blocks * a.ntt : 0.0);
+                        (sk ? 4.0 + (group == 64 ? 2.5 : 2.0) * 1024 / 4e6 * a.P * blocks * a.ntt : 0.0);
       if (us < best_us) best_us = us, best = t;
     }
   return best;
