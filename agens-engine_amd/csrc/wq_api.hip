@@ -25,6 +25,7 @@ int i8_gemv_m1(int bits, const void* x, int m, const Segs& g, int k, int group, 
 int i8_gemv_mt(int bits, const void* x, int m, const Segs& g, int k, int group, hipStream_t s, int act = 0);
 int tile_gemv(int bits, const void* x, int m, const Segs& g, int k, int group, hipStream_t s, int act);
 int mm_gemv(int bits, const void* x, int m, const Segs& g, int k, int group, hipStream_t s, int act);
+int num_cus();
 int m1d_chain_make(int nsteps, const int* bits, const void* const* x, const int* m, const int* k, const Segs* segs,
                    const int* wait, const int* act, void** table, int* mt_out, size_t* smem_out);
 int m1d_chain_launch(const void* table, int nsteps, int mt, size_t smem, hipStream_t s);
@@ -56,9 +57,10 @@ bool exact_mode() {
 }
 
 // The smallest token count routed to the fp16-MFMA kernel (wq_mm.hip) in the default numerics, where the tiled kernel
-// (tile_route) does not take the call: the measured crossover with the integer-limb kernels (below it those are faster).  Both compute the same numerics bit for bit, so the
-// switch changes speed only.  0: never; set through ak_wq_set_mm_min or AGENS_WQ_MM_MIN.  Above kMmMaxK inputs the
-// integer kernels stay faster at every token count (measured: down 5120 x 27648 at 24..128 tokens).
+// (tile_route) does not take the call: the measured crossover with the integer-limb kernels (below it those are faster).
+// Both compute the same numerics bit for bit, so the switch changes speed only.  0: never; set through ak_wq_set_mm_min
+// or AGENS_WQ_MM_MIN.  Above kMmMaxK inputs the integer kernels stay faster at every token count (measured: down 5120 x
+// 27648 at 24..128 tokens).
 constexpr int kMmMinDefault = 17;
 constexpr int kMmMaxK = 8192;
 std::atomic<int> g_mm_min{-1};
@@ -84,11 +86,32 @@ bool mm_route(int m, int k, int group, bool exact) {
   return m >= kMmMinDefault && k <= kMmMaxK;
 }
 
+// Group 64 at one and two tokens: whether the any-m kernel (wq_i8.hip) is the faster one.  Its workgroups own 64 rows and
+// all inputs, a wave per stripe, two workgroups per CU: a round of them takes about as long however full it is, and up to
+// 8 tiles of 1024 inputs hardly longer for more inputs.  The tiled kernel's time is proportional to both.  So the line is
+// where a round (or its half with one workgroup per CU) is well filled.  Measured (us, any-m / tiled, 1 token):
+//   second half of a round: 32768 x 8192 W4 42 / 58, 29000 x 5120 34 / 37, 23500 x 6144 W2 35 / 38, but 21000 x 6144 37 /
+//     31, 23500 x 5120 33 / 30; 2 tokens 32768 x 8192 W4 44 / 58, 26000 x 8192 44 / 46, 21000 x 8192 43 / 42;
+//   9 tiles and more (two tiles per wave: the any-m kernel's step up): 32768 x 10240 W2 59 / 68, 17500 x 9216 52 / 58, but
+//     17500 x 12288 60 / 55; 2 tokens 26000 x 10240 96 / 66 (one workgroup per CU: the activations' LDS);
+//   first half: 15000 x 5120 W4 27 / 29, W3 33 / 35, W2 26 / 26, 11000 x 5120 W4 26 / 22;
+//   third round, from its first half on: 98304 x 8192 W4 117 / 130, 82000 x 8192 110 / 124; the tiled kernel at 57000,
+//     65536 and 115000 rows (78 / 75, 80 / 78, 148 / 131).
+bool any_m_route(int bits, int m, const Segs& g, int k) {
+  if (m > 2) return false;
+  const int cus = num_cus(), wg = (g.end[g.nseg - 1] + 63) / 64, tiles = kpad(k) / 1024;
+  if (wg <= cus) return m == 1 && bits >= 3 && tiles >= 5 && tiles <= 6 && wg >= 4 * cus / 5;
+  if (wg <= 2 * cus) {
+    if (tiles <= 8) return tiles >= 5 && (long long)2 * wg * tiles >= 17 * cus && (m == 1 || 2 * wg >= 3 * cus);
+    return m == 1 && tiles <= 14 && wg >= cus + cus / 8 * (tiles - 9);
+  }
+  return m == 1 && tiles >= 7 && tiles <= 8 && wg > 4 * cus && wg <= 6 * cus;
+}
+
 // Whether a default-numerics call takes the tiled kernel (wq_tile.hip; same bits).  An explicit crossover keeps the older
 // kernels.  Measured, the older kernels' time -> the tiled kernel's, us:
-//   group 64 (which the small-M kernels do not take), every token count: 5120 x 6144 W4 28 -> 18 at 1 token, 188 -> 19 at
-//     16; 55296 x 5120 W3 84 -> 66 and 624 -> 70; 152064 x 5120 W4 153 -> 127 at 1; 22000 x 2560 W3 34.1 -> 33.9 at 1
-//     (the smallest gain met); 64 x 64 14.8 -> 11.1;
+//   group 64 (which the small-M kernels do not take), every token count but for any_m_route: 5120 x 6144 W4 28 -> 18 at 1
+//     token, 188 -> 19 at 16; 55296 x 5120 W3 84 -> 66 and 624 -> 70; 152064 x 5120 W4 153 -> 127 at 1; 64 x 64 14.8 -> 11.1;
 //   group 128 from 33 tokens: 55296 x 5120 W3 164 -> 86 at 64 tokens, 5120 x 5120 W4 38.6 -> 28.9, 5120 x 27648 W3 130 ->
 //     68, 64 x 512 19.8 -> 12.3; at 17 to 32 tokens on wide linears, 55296 x 5120 W3 82 -> 60, 14000 x 2560 W3 29.4 -> 22,
 //     7168 x 5120 W4 25.9 -> 24.2 at 17, but 5120 x 5120 W4 19.7 -> 20.4 and 1000 x 2048 W3 12.5 -> 13.6: the fp16-MFMA
@@ -96,14 +119,14 @@ bool mm_route(int m, int k, int group, bool exact) {
 //     tokens, from 24: 5120 x 27648 W2 51.9 -> 47.4 at 24, 45.5 -> 47.3 at 20;
 //   up to 16 tokens at group 128 the small-M kernels (55296 x 5120 W3, 16 tokens: 46 against 49).
 constexpr int kTileRows = 6144;
-bool tile_route(int m, const Segs& g, int k, int group, bool exact) {
+bool tile_route(int bits, int m, const Segs& g, int k, int group, bool exact) {
   if (exact || mm_min_set() >= 0) return false;
-  if (group == 64 || m > 32) return true;
+  if (group == 64) return !any_m_route(bits, m, g, k);
   if (m <= 16) return false;
-  if (k > kMmMaxK) return m >= 24;
   long long rows = 0;
   for (int i = 0; i < g.nseg; ++i) rows += g.n[i];
-  return rows > kTileRows;
+  if (k > kMmMaxK) return m >= 24;
+  return m > 32 || rows > kTileRows;
 }
 
 bool group_ok(int k, int group) { return (group == 64 || group == 128) && k % group == 0 && k % 32 == 0; }
@@ -179,7 +202,7 @@ int gemv(int bits, const void* x, int m, int nseg, const void* const* wt, const 
   if (act && exact) return AK_INVALID;  // the fused activation is in the default path's kernels only
   std::lock_guard<std::mutex> lock(scratch_mutex(s));
   const Segs all = make_segs(nseg, wt, st, y, n, ldy, 16);
-  if (tile_route(m, all, k, group, exact)) {
+  if (tile_route(bits, m, all, k, group, exact)) {
     const int e = tile_gemv(bits, x, m, all, k, group, s, act);
     if (e != AK_INVALID) return e;
   }
@@ -336,11 +359,11 @@ int ak_wq_gemv_kt_multi(int bits, const void* x, int m, int nseg, const void* co
   return gemv(bits, x, m, nseg, wt, st, y, n, ldy, k, group, bf16w, false, static_cast<hipStream_t>(stream));
 }
 
-// ak_wq_gemv_kt_multi that allocates nothing (no counterpart in the reference; for callers that cannot allocate:
-// code under stream capture, tight serving loops): its split-K launches use the library's static 64 MiB device
-// array instead of per-stream scratch.  1 (invalid value) when the call's worst-case split-K scratch
-// (noalloc_scratch_need) exceeds it, e.g. a 152064-row linear at 16 tokens.  Calls on one device share the array:
-// calls that overlap in time on one device race.
+// ak_wq_gemv_kt_multi that allocates nothing (no counterpart in the reference; for callers that cannot allocate: code
+// under stream capture, tight serving loops): its split-K partials and the tiled kernel's converted activations lie in
+// the library's static 64 MiB device array instead of library scratch.  1 (invalid value) when the call's worst-case
+// split-K scratch (noalloc_scratch_need) exceeds it, e.g. a 152064-row linear at 16 tokens.  Calls on one device share
+// the array: calls that overlap in time on one device race.
 int ak_wq_gemv_kt_multi_noalloc(int bits, const void* x, int m, int nseg, const void* const* wt, const void* const* st,
                                 void* const* y, const int* n, const int* ldy, int k, int group, int bf16w,
                                 void* stream) {

@@ -72,6 +72,19 @@ def test_wide_linears_equal_oracle(group, bits, m, n):
     assert_equals_oracle(y, x, m, L, [(0, 130), (n // 2, n // 2 + 130), (n - 130, n)])
 
 
+# both sides of the lines between the tiled kernel and the integer kernels (by full rounds of the latter's workgroups of
+# 64 rows at group 64)
+@pytest.mark.parametrize("group,bits,m,n,k", [(64, 4, 1, 13040, 5120), (64, 4, 1, 13057, 5120), (64, 3, 1, 16384, 5184),
+                                            (64, 2, 1, 32768, 5120), (64, 2, 1, 32769, 5120), (64, 3, 2, 24560, 6144),
+                                            (64, 3, 2, 24576, 6144), (64, 2, 1, 16400, 8256), (64, 4, 1, 65600, 6208)])
+def test_routes_equal_oracle(group, bits, m, n, k):
+    L = make(17, n, k, group, bits)
+    x = gen_x(19 + m, m * k)
+    (Y,) = gemv(bits, Dev.of(x), m, [L], k, group)
+    y = Y.get(np.uint16, m * n).reshape(m, n)
+    assert_equals_oracle(y, x, m, L, [(0, 40), (n // 2, n // 2 + 40), (n - 40, n)])
+
+
 @pytest.mark.parametrize("group,bits,m,n,k", [(128, 3, 40, 7000, 1024), (128, 2, 100, 600, 9344), (64, 4, 3, 600, 2112),
                                               (128, 2, 128, 40, 163840)])
 def test_equals_the_other_kernels(group, bits, m, n, k):
