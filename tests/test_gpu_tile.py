@@ -73,10 +73,11 @@ def test_wide_linears_equal_oracle(group, bits, m, n):
 
 
 # both sides of the lines between the tiled kernel and the integer kernels (by full rounds of the latter's workgroups of
-# 64 rows at group 64)
+# 64 rows at group 64; above 8192 inputs at group 128)
 @pytest.mark.parametrize("group,bits,m,n,k", [(64, 4, 1, 13040, 5120), (64, 4, 1, 13057, 5120), (64, 3, 1, 16384, 5184),
                                             (64, 2, 1, 32768, 5120), (64, 2, 1, 32769, 5120), (64, 3, 2, 24560, 6144),
-                                            (64, 3, 2, 24576, 6144), (64, 2, 1, 16400, 8256), (64, 4, 1, 65600, 6208)])
+                                            (64, 3, 2, 24576, 6144), (64, 2, 1, 16400, 8256), (64, 4, 1, 65600, 6208),
+                                            (128, 2, 33, 16001, 10368), (128, 3, 41, 16001, 10368)])
 def test_routes_equal_oracle(group, bits, m, n, k):
     L = make(17, n, k, group, bits)
     x = gen_x(19 + m, m * k)
