@@ -27,11 +27,13 @@ int ak_wq_tune_query(int bits, int m, int nseg, const int* n, int k, int* split,
  * splits' partial sums take.  0, or 1 for a shape that the call refuses. */
 int ak_wq_gemm_tune_query(int m, int n, int k, int* rows, int* tokens, int* splits, size_t* scratch);
 
-/* The smallest token count (m) that ak_wq_gemv_kt_multi and its conveniences route to the fp16-MFMA kernel in the
- * default numerics (group 128): m >= this many tokens take it, fewer take the integer-limb kernels, at every k.  0:
- * never (the integer-limb kernels for every m); negative: the compiled-in measured rule (17 tokens and k <= 8192; or
- * the environment variable AGENS_WQ_MM_MIN).  Both kernels compute the same numerics bit for bit, so this changes
- * speed only.  Process-wide.  Always 0. */
+/* An explicit crossover between the older kernels of the default numerics, for every ak_wq_gemv_kt_multi call: at group
+ * 128, m >= this many tokens take the fp16-MFMA kernel and fewer the integer-limb kernels, at every k; 0: the
+ * integer-limb kernels for every m.  While one is set (a value of 0 or more, or the environment variable
+ * AGENS_WQ_MM_MIN), the tiled kernel (csrc/wq_tile.h) is off at every group and token count -- also with the value 17,
+ * and also at group 64, where the any-m kernel is left: up to ten times slower (16 tokens, 5120 x 6144: 188 against 19
+ * us).  Negative: the compiled-in measured rules (tile_route, any_m_route and mm_route of csrc/wq_api.hip).  All of these
+ * kernels compute the same numerics bit for bit, so this changes speed only.  Process-wide.  Always 0. */
 int ak_wq_set_mm_min(int m);
 
 #ifdef __cplusplus

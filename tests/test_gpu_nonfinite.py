@@ -140,3 +140,38 @@ def test_nonfinite_on_the_mfma_route(bits, n, k, m):
     what = f"MFMA route bits={bits} n={n} k={k} m={m}"
     same_bits_nan_aware(ys[2], ora_fast(bits, x, m, wt, st, n, k, 128), what)
     same_bits_nan_aware(ys[2], ys[0], what + " vs the integer kernels")
+
+
+# the kernel that callers get at group 64 and above 16 tokens (csrc/wq_tile.h): one and several token tiles, k unsplit and
+# split (more than one 1024-input tile on few rows), the last group before the padding of k (k % 1024 != 0)
+TILED = [(4, 64, 96, 3072, 1), (3, 64, 256, 1088, 4), (2, 64, 130, 4160, 17), (4, 64, 20000, 1024, 4),
+         (2, 128, 300, 5120, 33), (3, 128, 96, 9344, 65), (4, 128, 6200, 1152, 17), (3, 128, 14000, 1024, 33),
+         (4, 128, 70, 640, 128), (2, 64, 9000, 320, 100)]
+
+
+@pytest.mark.parametrize("bits,group,n,k,m", TILED)
+def test_nonfinite_on_the_default_route(bits, group, n, k, m):
+    """The same activations with no crossover set: the oracle's bits, and what the integer kernels give."""
+    K = kernels()
+    lo, span = -(1 << (bits - 1)), 1 << bits
+    packed = gen_container(7400 + bits, n, k, lo, span)
+    scales = gen_scales(7401 + bits, n * k // group)
+    L = Linear(packed, scales, n, k, group, bits)
+    check(L.rc)
+    wt, st = L.host_kt()
+    x = special_x(m, k, group, 7500 + m)
+    X = Dev.of(x)
+    ys = {}
+    for mmin in (-1, 0):
+        K.ak_wq_set_mm_min(mmin)
+        try:
+            (Y,) = gemv(bits, X, m, [L], k, group)
+        finally:
+            K.ak_wq_set_mm_min(0)
+        ys[mmin] = Y.get(np.uint16, m * n).reshape(m, n)
+    what = f"default route bits={bits} g={group} n={n} k={k} m={m}"
+    same_bits_nan_aware(ys[-1], ys[0], what + " vs the integer kernels")
+    rows = (0, min(n, 300))
+    same_bits_nan_aware(ys[-1][:, :rows[1]], ora_fast(bits, x, m, wt, st, n, k, group, rows=rows)[:, :rows[1]], what)
+    for t in range(1, m, 4):
+        assert np.all(np.isnan(bf2f_array(ys[-1][t]))), f"{what}: a NaN input leaves every output NaN"

@@ -74,3 +74,14 @@ def test_ragged_shape_matches_oracle(i, mode):
         assert np.array_equal(got[:, :L.n], want), f"case {i}: segment of {L.n} rows differs"
         assert np.all(got[:, L.n:] == 0x7FC1), f"case {i}: writes past the segment's rows"
     K.ak_w4_set_mma(1)
+
+
+@pytest.mark.parametrize("i", [i for i, c in enumerate(CASES) if c[1] == 64 or c[3] > 16])
+def test_ragged_shape_on_the_default_route(i):
+    """The cases that callers who set no crossover see on the tiled kernel (group 64, more than 16 tokens)."""
+    K = kernels()
+    K.ak_wq_set_mm_min(-1)
+    try:
+        test_ragged_shape_matches_oracle(i, "default")
+    finally:
+        K.ak_wq_set_mm_min(0)

@@ -121,3 +121,31 @@ def test_noalloc_refuses_beyond_its_scratch():
                                         int_array([n]), None, k, 128, 0, None)
     assert rc == 1
     check(K.ak_synchronize())
+
+
+@pytest.mark.parametrize("bits,group,m,n,k", [(4, 64, 3, 600, 6144), (3, 128, 40, 7000, 1024), (2, 128, 64, 600, 9344)])
+def test_noalloc_on_the_default_route(bits, group, m, n, k):
+    """With no crossover set: the tiled kernel in the static array, twice in a row; free device memory unchanged."""
+    K = kernels()
+    L = Linear(gen_container(9300, n, k, -(1 << (bits - 1)), 1 << bits), gen_scales(9301, n * k // group), n, k, group, bits)
+    check(L.rc)
+    X, want, got = Dev.of(gen_x(9302, m * k)), Dev(m * n * 2), Dev(m * n * 2)
+
+    def run(fn, y):
+        return getattr(K, fn)(bits, X.p, m, 1, ptr_array([L.wt.p]), ptr_array([L.st.p]), ptr_array([y.p]),
+                              int_array([n]), None, k, group, 0, None)
+
+    check(run("ak_wq_gemv_kt_multi", want))  # the integer kernels
+    check(run("ak_wq_gemv_kt_multi_noalloc", got))
+    K.ak_wq_set_mm_min(-1)
+    try:
+        for _ in range(2):
+            check(K.ak_memcpy_h2d(got.p, np.full(m * n, 0x7FC1, dtype=np.uint16).ctypes.data, m * n * 2))
+            check(K.ak_synchronize())
+            before = free_mem()
+            check(run("ak_wq_gemv_kt_multi_noalloc", got))
+            check(K.ak_synchronize())
+            assert free_mem() == before
+            assert np.array_equal(got.get(np.uint16, m * n), want.get(np.uint16, m * n))
+    finally:
+        K.ak_wq_set_mm_min(0)
