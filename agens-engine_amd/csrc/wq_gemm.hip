@@ -391,7 +391,7 @@ int launch_tiles(const void* x, int m, const void* wt, const void* st, void* y, 
 // The tiling of a launch: T tokens per tile and the number of k splits, by the estimated time
 //   rounds x (slabs x slab time(R, T) + 3) + (split: 5 + the fp32 partials written and read at 8 TB/s) us,
 // rounds = workgroups per XCD / CUs per XCD, rounded up (one workgroup per CU at a time: at T = 64 two fit, but share
-// the same throughput).  Slab times measured at 240 workgroups (us): 0.65 at 128 x 128, 0.78 at 256 rows x 64 tokens, 1.12
+// the same throughput).  Slab times measured at 240 workgroups (us): 0.7 at 128 x 128, 0.78 at 256 rows x 64 tokens, 1.12
 // at 128, 1.42 at 192, 1.75 at 256 (the dequantization and the weight tile's LDS traffic do not shrink with T).  So wide
 // linears take the largest tile that does not pad too many tokens, and narrow or short ones the smallest, with k split
 // until one round is nearly full.  Measured
@@ -412,7 +412,7 @@ Tiling pick_tiling(int m, int n, int nslab, bool may_split) {
     static const struct {
       int R, T;
       double slab;
-    } kTiles[5] = {{128, 128, 0.65}, {256, 64, 0.78}, {256, 128, 1.12}, {256, 192, 1.42}, {256, 256, 1.75}};
+    } kTiles[5] = {{128, 128, 0.7}, {256, 64, 0.78}, {256, 128, 1.12}, {256, 192, 1.42}, {256, 256, 1.75}};
     for (int sp = 1; sp <= (may_split ? 32 : 1) && (sp == 1 || nslab / sp >= 4); ++sp) {
       const Tiling t = {kTiles[c].R, kTiles[c].T, sp};
       if (sp > 1 && part_bytes(t, m, n) > kMaxCallScratch) break;
