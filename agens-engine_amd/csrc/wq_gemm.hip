@@ -301,43 +301,55 @@ __global__ void __launch_bounds__(2 * R, R == 128 ? 2 : T == 64 ? 4 : 1) wq_gemm
   if (sl < nslab) body(sl, std::integral_constant<int, 0>());
   __builtin_amdgcn_s_waitcnt(kVmcnt0);  // no load into LDS outlives the workgroup
 
-  // 4 rows of a lane's output in one 8-byte store where the rows stay aligned
+  // D: register 4 g + e of lane l holds row 8 g + 4 (l / 32) + e of its 32-row tile for token l % 32.  4 rows of a lane's
+  // output go in one 8-byte store where the rows stay aligned; else they pass through the wave's share of the LDS, from
+  // where the wave writes a token's 64 rows at a time (a lane's own 2-byte stores fall on 32 tokens' rows: 45850 x 1792 W2
+  // at 256 tokens 77 us, so 55)
   const bool vec = ((n | ldy) & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 7) == 0;
-  // D: register 4 g + e of lane l holds row 8 g + 4 (l / 32) + e of its 32-row tile for token l % 32
+  uint8_t* const out = lds + wave * (T * 64);  // [T / 2 tokens][64 rows]: the 8-byte piece c of token t at slot c ^ (t & 15)
+  if constexpr (!SPLIT)
+    if (!vec) __syncthreads();  // every wave's loads into LDS have landed and its operands are read
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    const int t = t0 + wtk + 32 * j + l32;
+    const int tk = 32 * j + l32, t = t0 + wtk + tk;
     if (t >= m) continue;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int r0 = o0 + wr + 32 * i + 8 * g + 4 * hi;
         if constexpr (SPLIT) {
           reinterpret_cast<f32x4*>(part)[((size_t)item * (8 * NW * NJ) + ((wave * NJ + j) * 2 + i) * 4 + g) * 64 + lane] =
               f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
         } else {
-          uint16_t* yr = y + (size_t)t * ldy;
+          const int c = 8 * i + 2 * g + hi, r0 = o0 + wr + 4 * c;
           const bf16x2 lo = {(__bf16)acc[i][j][4 * g], (__bf16)acc[i][j][4 * g + 1]};
           const bf16x2 up = {(__bf16)acc[i][j][4 * g + 2], (__bf16)acc[i][j][4 * g + 3]};
-          if (vec) {
-            if (r0 < n)
-              *reinterpret_cast<uint2*>(yr + r0) =
-                  make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, up));
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (r0 + e < n) yr[r0 + e] = __builtin_bit_cast(uint16_t, (__bf16)acc[i][j][4 * g + e]);
-          }
+          const uint2 v = make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, up));
+          if (!vec)
+            *reinterpret_cast<uint2*>(out + tk * 128 + ((c ^ (tk & 15)) << 3)) = v;
+          else if (r0 < n)
+            *reinterpret_cast<uint2*>(y + (size_t)t * ldy + r0) = v;
         }
       }
   }
+  if constexpr (!SPLIT)
+    if (!vec) {
+      __syncthreads();
+      const int r = o0 + wr + lane, tokens = m - t0 - wtk < T / 2 ? m - t0 - wtk : T / 2;
+      if (r < n)
+#pragma unroll 8
+        for (int tk = 0; tk < tokens; ++tk)
+          y[(size_t)(t0 + wtk + tk) * ldy + r] =
+              *reinterpret_cast<const uint16_t*>(out + tk * 128 + (((lane >> 2) ^ (tk & 15)) << 3) + 2 * (lane & 3));
+    }
 }
 
 // y = bf16 of the splits' partials added in order.  A split's partials of a tile lie as its waves hold them (16 bytes per
 // lane: 4 rows of one token; R T / 256 such kilobytes per tile), so that they are written and read in whole lines; a
 // thread sums one 16-byte piece.  Eight splits' loads are requested before their sums (splits past the last one read the last
-// one again and are not added): one memory round trip per eight splits instead of one per split.
+// one again and are not added): one memory round trip per eight splits instead of one per split.  A workgroup's four
+// kilobytes are 32 rows of 32 tokens: where a lane's 4 outputs are no aligned 8 bytes, they pass through LDS, from where a
+// token's 32 rows are written side by side.
 __global__ void __launch_bounds__(256) sum_splits_kernel(const f32x4* __restrict__ part, int nsplit, int m, int n,
                                                          uint16_t* __restrict__ y, int ldy, int nrow_tiles, int tiles,
                                                          int R, int nj) {
@@ -345,9 +357,10 @@ __global__ void __launch_bounds__(256) sum_splits_kernel(const f32x4* __restrict
   const int tile = blockIdx.y, tt = tile / nrow_tiles, rt = tile - tt * nrow_tiles;
   const int wj = f >> 3, wave = wj / nj, j = wj - wave * nj;
   const int rw = R >> 6, wt = wave / rw;  // waves along the rows; the wave along the tokens
-  const int t = (tt * 2 + wt) * 32 * nj + 32 * j + (lane & 31);
-  const int o = rt * R + (wave - wt * rw) * 64 + 8 * (f & 7) + 4 * (lane >> 5);
-  if (t >= m || o >= n) return;
+  const int tb = (tt * 2 + wt) * 32 * nj + 32 * j, ob = rt * R + (wave - wt * rw) * 64 + 32 * ((f >> 2) & 1);
+  const int t = tb + (lane & 31), o = ob + 8 * (f & 3) + 4 * (lane >> 5);
+  const bool vec = ((n | ldy) & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 7) == 0;  // y may be a column offset
+  if (vec && (t >= m || o >= n)) return;
   const int kb = R * nj >> 2;  // kilobytes of a tile
   const f32x4* p = part + ((size_t)tile * kb + f) * 64 + lane;
   const size_t step = (size_t)tiles * kb * 64;
@@ -361,13 +374,20 @@ __global__ void __launch_bounds__(256) sum_splits_kernel(const f32x4* __restrict
       if (s0 + i < nsplit) acc += v[i];
   }
   const bf16x2 lo = {(__bf16)acc[0], (__bf16)acc[1]}, hi = {(__bf16)acc[2], (__bf16)acc[3]};
-  uint16_t* yo = y + (size_t)t * ldy + o;
-  if (o + 4 <= n && (ldy & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 7) == 0) {  // y may be a column offset
-    *reinterpret_cast<uint2*>(yo) = make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
-  } else {
+  const uint2 v = make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
+  if (vec) {
+    *reinterpret_cast<uint2*>(y + (size_t)t * ldy + o) = v;
+    return;
+  }
+  __shared__ uint32_t out[32][17];  // [token][32 rows as pairs]
+  out[lane & 31][(o - ob) >> 1] = v.x;
+  out[lane & 31][((o - ob) >> 1) + 1] = v.y;
+  __syncthreads();
+  const int r = threadIdx.x & 31;
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (o + e < n) yo[e] = __builtin_bit_cast(uint16_t, (__bf16)acc[e]);
+  for (int q = 0; q < 4; ++q) {
+    const int tk = (threadIdx.x >> 5) + 8 * q;
+    if (tb + tk < m && ob + r < n) y[(size_t)(tb + tk) * ldy + ob + r] = (uint16_t)(out[tk][r >> 1] >> (16 * (r & 1)));
   }
 }
 
