@@ -289,13 +289,16 @@ extern "C" int ak_i8_gemv(const void* x, const void* w, const void* scale, void*
   // kernel where one part covers them, or two.  Measured (us, 152064 x 5120, before = activations from L1 per token and
   // row pair): 2 / 4 / 8 / 16 tokens 156 / 233 / 358 / 628 -> 119 / 148 / 228 / 460.  Two or three tokens on less than 32
   // MB of weights stay with the kernel below (8001 x 1040: 7.1 against 7.4, 7.4 against 7.7).
-  // The second part reads all weights again.  Below 32 MB they are still in the caches (1700 x 16400, 4 tokens 50.9 ->
-  // 44.2; 1700 x 13648, 6 tokens 55.5 -> 41.8); above, it pays only for parts of up to four tokens or more (60000 x 10240,
-  // 8 tokens 294 -> 267; 33000 x 8192, 9 tokens 176 -> 136), not for less (12000 x 24576, 2 tokens 73 against 104; 12000 x
-  // 16400, 4 tokens 78 against 97; 60000 x 12288, 6 tokens 319 against 338).
+  // The second part reads all weights again.  Below 80 MB the caches still hold most of them, and four tokens or more gain
+  // (1700 x 20480, 4 tokens 61.8 -> 53.8; 6000 x 13648, 6 tokens 64.8 -> 49.9; but 6000 x 16400, 94 MB, 4 tokens 52.7 ->
+  // 54.9); above, it pays only for parts of up to four tokens or more (60000 x 10240, 8 tokens 294 -> 267; 33000 x 8192, 9
+  // tokens 176 -> 136), not for less (12000 x 24576, 2 tokens 73 against 104; 12000 x 16400, 4 tokens 78 against 97; 60000
+  // x 12288, 6 tokens 319 against 338).
   const int cap = 40960 / k, most = cap < 8 ? cap : 8;
-  const bool small = (long long)n * k < 32 << 20;
-  if (most > 0 && (small ? m > 3 && m <= 2 * most : m > 1 && m <= (most < 4 ? most : 2 * most))) {
+  const long long bytes = (long long)n * k;
+  const bool one = m > 1 && m <= most && (m > 3 || bytes >= 32 << 20);
+  const bool two = m > 3 && m > most && m <= 2 * most && (most >= 4 || bytes < 80 << 20);
+  if (one || two) {
     const int parts = (m + most - 1) / most, per = (m + parts - 1) / parts;
     for (int m0 = 0; m0 < m; m0 += per)
       agq::lds_part(X + (size_t)m0 * k, W, S, Y + (size_t)m0 * ldy, m - m0 < per ? m - m0 : per, n, k, ldy, s);

@@ -50,10 +50,10 @@ def test_matches_oracle_bit_exact(m, n, k):
                                    (7, 32769, 144), (8, 32770, 2064), (2, 2049, 16400), (4, 515, 5120), (6, 31, 48),
                                    (7, 300, 1040), (8, 1, 5120), (11, 40, 5120), (13, 32775, 528), (16, 97, 4112),
                                    (16, 40, 5136), (3, 33, 20496),
-                                   # the line of the second part: below and above 32 MB of weights, parts of up to 1,
-                                   # 2, 3 and 4 tokens
-                                   (2, 1640, 20496), (3, 2047, 16400), (4, 2045, 16400), (4, 2047, 16400),
-                                   (6, 3271, 10256), (6, 3272, 10256), (7, 4100, 8208)])
+                                   # the lines of the second part: parts of up to 1, 2, 3 and 4 tokens, below and
+                                   # above 80 MB of weights
+                                   (2, 1640, 20496), (3, 2047, 16400), (4, 2047, 16400), (4, 5114, 16400),
+                                   (4, 5116, 16400), (6, 8179, 10256), (6, 8180, 10256), (7, 4100, 8208)])
 def test_tokens_in_lds_match_oracle_bit_exact(m, n, k):
     x, q, scale = data(40 + m + n, m, n, k)
     ldy = n + 3
