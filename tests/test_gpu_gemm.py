@@ -156,13 +156,13 @@ def test_gemm_wide_tiles_exact_on_small_integer_operands(bits):
     (4, 64, 192, 40001, 64), (2, 128, 193, 40000, 384), (3, 64, 256, 40001, 192),
     (2, 128, 1, 257, 2304), (4, 64, 64, 255, 1088), (3, 128, 65, 1, 4096), (4, 128, 129, 5120, 1152),
     (2, 64, 200, 2331, 2752), (3, 128, 333, 5117, 2304), (4, 128, 512, 2050, 1024)])
-def test_gemm_tilings_exact_on_small_integer_operands(bits, group, m, n, k):
+def test_gemm_tilings_exact_on_small_integer_operands(bits, group, m, n, k, pad=3):
     """Integer inputs and power-of-two scales: every product and partial sum is exact in fp32 (|sum| < 2^24 units of the
     smallest scale), so every output must equal the fp64 product rounded once to bf16."""
     L = make(8750 + bits + m, n, k, group, bits, scale_pow2=True)
     rng = np.random.default_rng(8751 + m)
     x = f2bf_array(rng.integers(-3, 4, (m, k)).astype(np.float32))
-    ld = n + 3
+    ld = n + pad
     y = gemm(L, Dev.of(x), m, ldy=ld, fill=0x7FC1)
     ref = bf2f_array(x).astype(np.float64) @ bf2f_array(dequant_host(L)).astype(np.float64).T
     assert np.array_equal(y[:, :n], f2bf_array(ref.astype(np.float32)))
@@ -170,7 +170,7 @@ def test_gemm_tilings_exact_on_small_integer_operands(bits, group, m, n, k):
 
 
 # (the tiling that the shape takes, rows x tokens, and whether k is split): the smaller tile at its edges, with few, odd
-# and many slabs, and the others split
+# and many slabs, and the others split; `aligned`: rows and their stride multiples of 4 (8-byte stores), else through LDS
 @pytest.mark.parametrize("bits,group,m,n,k,tile,split", [
     (4, 64, 127, 1, 64, (128, 128), False), (3, 128, 129, 385, 128, (128, 128), False),
     (2, 64, 130, 4097, 192, (128, 128), False), (4, 128, 1025, 1999, 128, (128, 128), False),
@@ -178,11 +178,13 @@ def test_gemm_tilings_exact_on_small_integer_operands(bits, group, m, n, k):
     (4, 64, 33, 1000, 4160, (256, 64), True), (3, 64, 64, 2331, 4160, (256, 64), True),
     (2, 64, 385, 5117, 4160, (256, 128), True), (4, 64, 129, 9999, 4160, (256, 192), True),
     (3, 64, 385, 9999, 4160, (256, 256), True)])
-def test_gemm_every_tile_exact_on_small_integer_operands(bits, group, m, n, k, tile, split):
+@pytest.mark.parametrize("aligned", [False, True])
+def test_gemm_every_tile_exact_on_small_integer_operands(bits, group, m, n, k, tile, split, aligned):
+    n = (n + 3) // 4 * 4 if aligned else n
     r, t, sp, nbytes = ctypes.c_int(), ctypes.c_int(), ctypes.c_int(), ctypes.c_size_t()
     assert kernels().ak_wq_gemm_tune_query(m, n, k, *[ctypes.byref(v) for v in (r, t, sp, nbytes)]) == 0
     assert (r.value, t.value) == tile and (sp.value > 1) == split
-    test_gemm_tilings_exact_on_small_integer_operands(bits, group, m, n, k)
+    test_gemm_tilings_exact_on_small_integer_operands(bits, group, m, n, k, pad=4 if aligned else 3)
 
 
 def test_split_k_gemm_leaves_gemv_scratch_intact():
