@@ -175,7 +175,9 @@ __device__ __forceinline__ float tile_group_sum(int d0, int d1, int d2) {
 __device__ __forceinline__ int tile_slot(int h, int r) { return h * 16 + (r ^ ((-4 * h) & 15)); }
 
 // RG x TW = 8 waves: wave = token tile (wave % TW), row group (wave / TW) of RB 16-row blocks.  NA: LDS stages of the
-// activation records; R: register sets of raw weights.  SK: workgroup = (row range, stripe).
+// activation records; R: register sets of raw weights.  SK: workgroup = (row range, stripe).  RB <= 2 is held to 128
+// registers so that two workgroups fit a CU (up to RB = 2 at 2, 3 and 5 token tiles of group 128; at 4 and 6 to 8 the LDS
+// holds one, and the bound only makes the unsplit kernels spill: W4 3 registers at RG = 2 and 15 at RG = 1, W3 1 and 4).
 template <int BITS, int G, int RG, int RB, bool SK>
 __global__ void __launch_bounds__(512, RB <= 2 ? 4 : 2) tile_kernel(const TileArgs a) {
   constexpr int NW = 8, NT = 512, TW = NW / RG, NA = tile_stages(RG), R = RB >= 5 ? 2 : 4;

@@ -18,7 +18,8 @@ int row_ranges(const Segs& g, int blocks) {  // workgroups that cover the segmen
 // The launch shape with the smallest estimated time (rb = 0: none fits).  Workgroups run in rounds of one per CU; a step
 // (one group of inputs) takes about 0.45 + 0.21 rb us at group 128 and three quarters of that at group 64 (measured us
 // per step, g128: 0.65 at 1 block per wave, 0.85 at 2, 1.25 at 4, 1.5 at 5, 1.95 at 7; g64: 0.52 at 1, 0.7 at 2, 1.4 at
-// 7), two workgroups of up to 2 blocks per wave share a CU at about 0.85 of the time.  A split takes as long as its
+// 7), two workgroups of up to 2 blocks per wave share a CU at about 0.85 of the time (applied to every such shape, also
+// where the LDS holds only one: group 128 and 2 blocks per wave at 4 and 6 to 8 token tiles).  A split takes as long as its
 // longest stripe, and adds its partials' traffic (2 us per 4 MB, 2.5 at group 64) and the last workgroups' sums: 9 tiles
 // are 2 per stripe, not 9 / 8 (20000 x 8320 W2, 33 tokens: split 132, unsplit 87; 90000 x 9216 W4 g64, 1 token: 211 and
 // 140), and many rows pay more for the partials than for another round (98304 x 8192 W4 g64, 1 token: split 151, unsplit

@@ -156,8 +156,8 @@ int ak_bf16_linear_f32reduce_ld(const void* x, const void* w, void* y, int m, in
  * bf16_linear.cu:68-80).  y[t][o] (row stride ldy; 0: n) = bf16(sum_i x[t][i] * w[o][i]) for every token t < m and
  * row o < n of a KT linear, w[o][i] = bf16_rn(q * scale) (the dequantized values, bit for bit), fp32 accumulation in
  * this kernel's order (within fp32-accumulation error of the two-call route); no weight copy.  Where the linear has
- * too few output tiles to fill the GPU, k is split across workgroups: fp32 partials in the stream's split-K scratch
- * (above), added in a fixed order by a second kernel, so results are deterministic for a given shape.  group in {64, 128}, k % group == 0, ldy >= n, else 1. */
+ * too few output tiles to fill the GPU, k is split across workgroups: fp32 partials in library scratch
+ * (above; inside a capture the graph's own), added in a fixed order by a second kernel, so results are deterministic for a given shape.  group in {64, 128}, k % group == 0, ldy >= n, else 1. */
 int ak_wq_gemm_kt(int bits, const void* x, int m, const void* wt, const void* st, void* y, int n, int ldy, int k,
                   int group, void* stream);
 
