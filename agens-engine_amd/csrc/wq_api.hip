@@ -117,10 +117,7 @@ bool any_m_route(int bits, int m, const Segs& g, int k) {
 //     7168 x 5120 W4 25.9 -> 24.2 at 17, but 5120 x 5120 W4 19.7 -> 20.4 and 1000 x 2048 W3 12.5 -> 13.6: the fp16-MFMA
 //     kernel up to kTileRows rows; past kMmMaxK inputs, where the other side is the integer kernels in chunks of 16
 //     tokens, from 24: 5120 x 27648 W2 51.9 -> 47.4 at 24, 45.5 -> 47.3 at 20;
-//     and not at 33 to 40 tokens on about 16000 to 24000 rows of 11 to 16 tiles, where the row ranges neither fill one
-//     round nor split well and the integer kernels' third chunk is a short one: 18000 x 13312 W2 99 -> 126 at 33, 100 ->
-//     128 at 36; 22000 x 14336 W3 129 -> 174 at 33 (but 22000 x 13312 0.96 of the integer kernels' time, 14000 x 13312
-//     88 -> 92, 28000 x 13312 0.8);
+//     and not where tile_gemv leaves 33 to 48 tokens of long k to the integer kernels (integer_kernels_faster);
 //   up to 16 tokens at group 128 the small-M kernels (55296 x 5120 W3, 16 tokens: 46 against 49).
 constexpr int kTileRows = 6144;
 bool tile_route(int bits, int m, const Segs& g, int k, int group, bool exact) {
@@ -129,11 +126,7 @@ bool tile_route(int bits, int m, const Segs& g, int k, int group, bool exact) {
   if (m <= 16) return false;
   long long rows = 0;
   for (int i = 0; i < g.nseg; ++i) rows += g.n[i];
-  if (k > kMmMaxK) {
-    const int tiles = kpad(k) / 1024;
-    const bool between = tiles >= 11 && tiles <= 16 && rows > 16000 && rows <= (tiles < 14 ? 20000 : 24000);
-    return m >= 24 && !(m > 32 && m <= 40 && between);
-  }
+  if (k > kMmMaxK) return m >= 24;
   return m > 32 || rows > kTileRows;
 }
 

@@ -51,6 +51,25 @@ TileShape pick_shape(const TileArgs& a, int group) {
   return best;
 }
 
+// 33 to 48 tokens at group 128 and k > 8192, where the other side is the integer kernels (wq_i8mt.hip) in chunks of 16
+// tokens.  A split launch of more than one round pays 5 to 8 us per round for its start and its partials, which counts
+// against stripes of one or two tiles of inputs.  Up to 40 tokens the integer kernels' third chunk is a short one: they are
+// faster from two rounds on, at W2 at longer stripes too, but for up to about 10000 rows, where the two are equal.  With a
+// full third chunk they are from three rounds on (not with SiLU, which each of their row ranges computes).  Measured (us,
+// tiled / integer): 33 tokens, 2 tiles per stripe 11000 x 10496 W4 89 / 73, 18000 x 12544 W3 135 / 113, 14000 x 14592 W2 90
+// / 87, 8192 x 10496 W4 61 / 58; 3 and 4 tiles 12288 x 19712 W2 116 / 108, W3 123 / 133, 18000 x 27648 W2 207 / 176, W4 212
+// / 237; unsplit 16000 x 10496 W2 73 / 87; 41 tokens 21927 x 13696 W2 155 / 138, 24218 x 14592 W3 172 / 176, 17335 x 11648 W2
+// 121 / 112; 42 tokens, two rounds 0.9 of the integer kernels' time, three rounds of 3 tiles 0.7 to 0.9.
+bool integer_kernels_faster(const TileArgs& a, const TileShape& t, int bits, int k, int group, int act) {
+  if (group != 128 || k <= 8192 || a.m <= 32 || a.m > 48 || !t.sk) return false;
+  const int workgroups = row_ranges(a.segs, t.rg * t.rb) * a.P, cus = num_cus();
+  const bool short_stripes = kpad(k) / 1024 <= 2 * a.P;
+  if (a.m > 40) return workgroups > 2 * cus && short_stripes && !act;
+  long long rows = 0;
+  for (int i = 0; i < a.segs.nseg; ++i) rows += a.segs.n[i];
+  return workgroups > cus && rows > 10240 && (bits == 2 || short_stripes);
+}
+
 }  // namespace
 
 // 1..128 tokens at group 64, 17..128 at group 128; act = 1 (group 128): x is the merged gate_up [m][2k] and the activations SiLU(gate) *
@@ -69,7 +88,7 @@ int tile_gemv(int bits, const void* x, int m, const Segs& g, int k, int group, h
     if ((long long)(kpad(k) / 1024) * g.n[i] * 128 * bits >= (1ll << 31)) return AK_INVALID;
   a.img_bytes = (size_t)(kpad(k) / group) * a.ntt * tile_rec_bytes(group);
   const TileShape t = pick_shape(a, group);
-  if (!t.rb) return AK_INVALID;
+  if (!t.rb || integer_kernels_faster(a, t, bits, k, group, act)) return AK_INVALID;
   size_t part = 0;
   if (t.sk)
     for (int i = 0; i < g.nseg; ++i) part += (size_t)a.P * a.ntt * ((g.n[i] + 15) / 16) * 1024;

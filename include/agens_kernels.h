@@ -23,8 +23,9 @@
  *     needs scratch, on any stream) that belongs to the captured graph: it may run beside other graphs and beside calls
  *     on the stream it was captured from (not beside itself).  Without a reserve, or with too little of it left, they
  *     take a launch that needs no scratch (the GEMV: same results; the GEMM: k not split).  The split-K launches of the
- *     one- to 16-token kernels at group 128 work in the captured stream's own scratch (if it has any): run graphs that
- *     hold such launches in order with each other and with calls on that stream.
+ *     one- to 16-token kernels at group 128, which some calls of more tokens take in chunks of 16, work in the captured
+ *     stream's own scratch (if it has any): run graphs that hold such launches in order with each other and with calls
+ *     on that stream.
  */
 #pragma once
 #include <stddef.h>
