@@ -115,11 +115,13 @@ bool any_m_route(int bits, int m, const Segs& g, int k) {
 //   group 128 from 33 tokens: 55296 x 5120 W3 164 -> 86 at 64 tokens, 5120 x 5120 W4 38.6 -> 28.9, 5120 x 27648 W3 130 ->
 //     68, 64 x 512 19.8 -> 12.3; at 17 to 32 tokens on wide linears, 55296 x 5120 W3 82 -> 60, 14000 x 2560 W3 29.4 -> 22,
 //     7168 x 5120 W4 25.9 -> 24.2 at 17, but 5120 x 5120 W4 19.7 -> 20.4 and 1000 x 2048 W3 12.5 -> 13.6: the fp16-MFMA
-//     kernel up to kTileRows rows; past kMmMaxK inputs, where the other side is the integer kernels in chunks of 16
+//     kernel up to kTileRows rows, at 3 tiles of inputs up to its one round of 8192 (kTileRows3: 6200 x 3072 W2 at 32
+//     tokens 15.8 -> 17.4, 7680 x 3072 W3 17.3 -> 18.2, 8208 x 3072 27.0 -> 17.7; 4 tiles 6200 rows 17.5 -> 18.1, 8192
+//     rows the same; 2 tiles 0.97); past kMmMaxK inputs, where the other side is the integer kernels in chunks of 16
 //     tokens, from 24: 5120 x 27648 W2 51.9 -> 47.4 at 24, 45.5 -> 47.3 at 20;
 //     and not where tile_gemv leaves 33 to 48 tokens of long k to the integer kernels (integer_kernels_faster);
 //   up to 16 tokens at group 128 the small-M kernels (55296 x 5120 W3, 16 tokens: 46 against 49).
-constexpr int kTileRows = 6144;
+constexpr int kTileRows = 6144, kTileRows3 = 8192;
 bool tile_route(int bits, int m, const Segs& g, int k, int group, bool exact) {
   if (exact || mm_min_set() >= 0) return false;
   if (group == 64) return !any_m_route(bits, m, g, k);
@@ -127,7 +129,7 @@ bool tile_route(int bits, int m, const Segs& g, int k, int group, bool exact) {
   long long rows = 0;
   for (int i = 0; i < g.nseg; ++i) rows += g.n[i];
   if (k > kMmMaxK) return m >= 24;
-  return m > 32 || rows > kTileRows;
+  return m > 32 || rows > (kpad(k) == 3072 ? kTileRows3 : kTileRows);
 }
 
 bool group_ok(int k, int group) { return (group == 64 || group == 128) && k % group == 0 && k % 32 == 0; }
