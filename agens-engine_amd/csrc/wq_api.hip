@@ -119,7 +119,7 @@ bool any_m_route(int bits, int m, const Segs& g, int k) {
 //     tokens 15.8 -> 17.4, 7680 x 3072 W3 17.3 -> 18.2, 8208 x 3072 27.0 -> 17.7; 4 tiles 6200 rows 17.5 -> 18.1, 8192
 //     rows the same; 2 tiles 0.97); past kMmMaxK inputs, where the other side is the integer kernels in chunks of 16
 //     tokens, from 24: 5120 x 27648 W2 51.9 -> 47.4 at 24, 45.5 -> 47.3 at 20;
-//     and not where tile_gemv leaves 33 to 48 tokens of long k to the integer kernels (integer_kernels_faster);
+//     and not where tile_gemv leaves 33 to 40 tokens of long k to the integer kernels (integer_kernels_faster);
 //   up to 16 tokens at group 128 the small-M kernels (55296 x 5120 W3, 16 tokens: 46 against 49).
 constexpr int kTileRows = 6144, kTileRows3 = 8192;
 bool tile_route(int bits, int m, const Segs& g, int k, int group, bool exact) {

@@ -80,7 +80,8 @@ def test_wide_linears_equal_oracle(group, bits, m, n):
                                             (128, 2, 33, 16001, 10368), (128, 3, 41, 16001, 10368),
                                             (128, 3, 33, 10240, 10368), (128, 3, 33, 10241, 10368), (128, 4, 40, 10241, 16384),
                                             (128, 4, 41, 10241, 16384), (128, 4, 33, 10241, 16512), (128, 2, 33, 10241, 16512),
-                                            (128, 2, 48, 16501, 10368), (128, 2, 49, 16501, 10368), (128, 3, 17, 8192, 2176), (128, 3, 32, 8193, 3072)])
+                                            (128, 2, 33, 17001, 10368), (128, 2, 41, 17001, 10368), (128, 3, 64, 12635, 6912),
+                                            (128, 2, 65, 22288, 6528), (128, 3, 17, 8192, 2176), (128, 3, 32, 8193, 3072)])
 def test_routes_equal_oracle(group, bits, m, n, k):
     L = make(17, n, k, group, bits)
     x = gen_x(19 + m, m * k)
